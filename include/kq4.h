@@ -116,8 +116,9 @@ const char *kq4_version(void);
  * gemv_wpcu, gemv_maxw, gemv_fq (0 / 1: activations quantized by a separate launch / in the
  * GEMV), gemv_fq_work, gemv_silu_fq_work, gemv_chunk_max (the largest q4 batch the decode GEMV
  * takes, 9..16 tokens in one launch of its 16-token kernel, 16 by default; 8 or less: every batch beyond 8 tokens
- * on the prefill GEMM; Q8_0 batches beyond 8 tokens always take the GEMM), gemm_kind (0: the prefill GEMM on int8 MFMA, the
- * default; 1: on fp8 operands; the same outputs), gemm_tile (0: the planner's choice; 1 / 2 / 3 /
+ * on the prefill GEMM; Q8_0 batches beyond 8 tokens always take the GEMM), gemm_kind (the form of the prefill GEMM's
+ * activations: 0 token-major, 1 as tile records where the chain has that form - ASM and Q8GEMM -,
+ * -1, the default, the planner's choice; the same outputs), gemm_tile (0: the planner's choice; 1 / 2 / 3 /
  * 4: 128x128 / 64x128 / 64x64 / 128x64 token x row tiles; the same outputs), gemm_split (K slices
  * of the int8 GEMM: 0 or 1 none, every output the single chain bit for bit; 2..8 that many;
  * -1 the planner's choice, the default), gemm_prio (the pipelined int8 GEMM's issue priority
@@ -134,8 +135,8 @@ int kq4_get_option(const char *name, int *value);
  * weights; chain as for kq4_matmul; ncu: the CUs to plan for, 0 = the current device's):
  * *tile = 0 and *ksplit = 0 for the decode GEMV (up to 8 tokens; q4 up to gemv_chunk_max), else the prefill
  * GEMM's tile (1 / 2 / 3 / 4: 128x128 / 64x128 / 64x64 / 128x64 tokens x rows) and its K
- * slices (1 = unsplit: the single chain, bit for bit); the int8 GEMM's plan (the fp8-operand
- * form of gemm_kind 1 picks its tile apart and never splits K). For tests and measurement; no
+ * slices (1 = unsplit: the single chain, bit for bit); the token-major form's plan (the
+ * record form keeps the K slices and may take another tile). For tests and measurement; no
  * counterpart in the reference. */
 int kq4_gemm_plan_info(int n_batch, int rows, int cols, int q8, int chain, int ncu, int *tile,
                        int *ksplit);

@@ -157,12 +157,12 @@ struct Carve {   // bump allocator over a workspace
   }
 };
 
-// Bytes of a matmul's quantized activations (int8 codes + f32 scales, token-major) in the
-// workspace, and of the fp8 GEMM's operand pairs (64 B per token and block) + scales.
+// Bytes of a matmul's quantized activations in the workspace (int8 codes + f32 scales, token-major).
 size_t qa_bytes(int n, int cols) {
   return al256((size_t)n * cols) + al256((size_t)n * (cols / 32) * sizeof(float));
 }
-size_t f8_bytes(int n, int cols) {
+// The operand bytes kq4_matmul_noalloc_dev's documented limit counts (17/8 of a byte per element).
+size_t noalloc_bytes(int n, int cols) {
   return al256((size_t)n * (cols / 32) * 64) + al256((size_t)n * (cols / 32) * sizeof(float));
 }
 
@@ -352,7 +352,7 @@ int run_gemv(DevState *ds, const Ws &wsp, int n_mats, float *const *out, const f
     } else {
       int8_t *q = cv.take<int8_t>((size_t)n * cols);
       float *d = cv.take<float>((size_t)n * nb);
-      KQ4_HIP((hipError_t)kq4_launch_quantize(x, q, d, nullptr, n, cols, 0, s, 0, xu));
+      KQ4_HIP((hipError_t)kq4_launch_quantize(x, q, d, nullptr, n, cols, 0, s, xu));
       xq = q;
       xd = d;
     }
@@ -377,6 +377,36 @@ int run_gemv(DevState *ds, const Ws &wsp, int n_mats, float *const *out, const f
     g += ((rows[i] + 31) / 32 + pl.rps - 1) / pl.rps << pl.hs;
   }
   KQ4_HIP((hipError_t)kq4_launch_gemv(a, n, kind, pl.hs, pl.rps, wgs, s));
+  return KQ4_OK;
+}
+
+// Whether a prefill GEMM of n tokens, planned as pl[], runs on activation records (kq4_gemm_rec.hip),
+// with each matrix's tile then in pl[]: option gemm_kind 0 never, 1 always, else where every matrix's
+// launch is faster so (kq4_rec_tile); the operands must stay within the kernel's buffer offsets and
+// the workspace hold the records and `more` bytes. A workspace that cannot grow to that (a fixed
+// buffer, a capturing stream) is no error: the call then takes the token-major form, which needs less
+// and gives the same bits.
+bool rec_fits(const DevState *ds, const Ws &ws, int n_mats, const int *rows, int cols, int n, int wf,
+              KQ4GemmPlan *pl, size_t more, hipStream_t s) {
+  const int kind = opt(kGemmKind);
+  int t[KQ4_MAX_MATS];
+  for (int i = 0; i < n_mats; ++i) {
+    t[i] = kind == 1 ? pl[i].tile : kq4_rec_tile(n, rows[i], wf, ds->ncu, pl[i]);
+    if (opt(kGemmTile) > 0 && t[i] != pl[i].tile) t[i] = 0;   // a forced tile is taken as it is
+    if (kind == 0 || !t[i] || !kq4_gemm_rec_ok(rows[i], cols, n, wf)) return false;
+  }
+  if (ensure_ws(ws, al256(kq4_rec_bytes(n, cols)) + more, s) != KQ4_OK) return false;
+  for (int i = 0; i < n_mats; ++i) pl[i].tile = t[i];
+  return true;
+}
+
+int rec_gemms(int n_mats, float *const *out, const float *const *res, const uint8_t *const *w,
+              const int *rows, int cols, int n, int wf, const uint8_t *rec, const KQ4GemmPlan *pl,
+              float *part, hipStream_t s) {
+  for (int i = 0; i < n_mats; ++i)
+    KQ4_HIP((hipError_t)kq4_launch_gemm_rec(out[i], res ? res[i] : nullptr, w[i], rec, rows[i], cols,
+                                            n, wf, s, pl[i].tile, pl[i].ksplit, part,
+                                            opt(kGemmPrio) != 0));
   return KQ4_OK;
 }
 
@@ -432,13 +462,20 @@ int matmul_impl(int n_mats, float *const *out, const float *const *res, const ui
     const int qc = gchain ? KQ4_CHAIN_Q8GEMM : KQ4_CHAIN_GEMV32;
     KQ4GemmPlan pl[KQ4_MAX_MATS];
     const size_t pbytes = split_bytes(n_mats, rows, cols, n, 1, qc, ds->ncu, pl);
+    if (x && gchain && rec_fits(ds, ws, n_mats, rows, cols, n, 1, pl, pbytes, s)) {
+      Carve cv{static_cast<char *>(ws.b->p)};
+      uint8_t *rec = cv.take<uint8_t>(kq4_rec_bytes(n, cols));
+      KQ4_HIP((hipError_t)kq4_launch_quantize_rec(x, nullptr, rec, nullptr, nullptr, n, n, cols, s));
+      return rec_gemms(n_mats, out, res, w, rows, cols, n, 1, rec, pl,
+                       pbytes ? cv.take<float>(pbytes / sizeof(float)) : nullptr, s);
+    }
     if ((rc = ensure_ws(ws, qbytes + pbytes, s))) return rc;
     Carve cv{static_cast<char *>(ws.b->p)};
     KQ4GemmAct act{xq_in, cols, 32, xd_in, nb, 1};
     if (x) {
       int8_t *q = cv.take<int8_t>((size_t)n * cols);
       float *d = cv.take<float>((size_t)n * nb);
-      KQ4_HIP((hipError_t)kq4_launch_quantize(x, q, d, nullptr, n, cols, 0, s, 0));
+      KQ4_HIP((hipError_t)kq4_launch_quantize(x, q, d, nullptr, n, cols, 0, s));
       act = KQ4GemmAct{q, cols, 32, d, nb, 1};
     } else {
       cv.off = qbytes;
@@ -459,19 +496,9 @@ int matmul_impl(int n_mats, float *const *out, const float *const *res, const ui
   const int main_n = chain == KQ4_CHAIN_AUTO ? (n & ~3) : n;
   const int tail = n - main_n;
   const int main_chain = chain == KQ4_CHAIN_AUTO ? KQ4_CHAIN_ASM : chain;
-  if (x && (main_chain == KQ4_CHAIN_ASM || main_chain == KQ4_CHAIN_GEMV32) && opt(kGemmKind) == 1) {
-    // fp8 operands (kq4_launch_gemm_f8): the main segment's activations quantized once into
-    // e4m3 operand pairs, the tail tokens by the GEMV from their fp32 rows
-    if ((rc = ensure_ws(ws, f8_bytes(main_n, cols), s))) return rc;
-    Carve cv{static_cast<char *>(ws.b->p)};
-    uint8_t *xp = cv.take<uint8_t>((size_t)main_n * nb * 64);
-    float *d = cv.take<float>((size_t)main_n * nb);
-    KQ4_HIP((hipError_t)kq4_launch_quantize(x, reinterpret_cast<int8_t *>(xp), d, nullptr, main_n,
-                                            cols, 0, s, 2, xu));
-    for (int i = 0; i < n_mats; ++i)
-      KQ4_HIP((hipError_t)kq4_launch_gemm_f8(out[i], res ? res[i] : nullptr, w[i], xp, d,
-                                             rows[i], cols, main_n, main_chain, ds->ncu, s,
-                                             opt(kGemmTile)));
+  KQ4GemmPlan pl[KQ4_MAX_MATS];
+  const size_t pbytes = split_bytes(n_mats, rows, cols, main_n, 0, main_chain, ds->ncu, pl);
+  auto tail_gemv = [&](const int8_t *tq, const float *td) -> int {
     if (!tail) return KQ4_OK;
     float *o2[KQ4_MAX_MATS];
     const float *r2[KQ4_MAX_MATS];
@@ -479,11 +506,39 @@ int matmul_impl(int n_mats, float *const *out, const float *const *res, const ui
       o2[i] = out[i] + (size_t)main_n * rows[i];
       r2[i] = (res && res[i]) ? res[i] + (size_t)main_n * rows[i] : nullptr;
     }
-    return run_gemv(ds, ws, n_mats, o2, r2, w, rows, cols, x + (size_t)main_n * cols,
-                    xu ? xu + (size_t)main_n * cols : nullptr, nullptr, nullptr, tail, 0, s);
+    return run_gemv(ds, ws, n_mats, o2, r2, w, rows, cols, nullptr, nullptr, tq, td, tail, 0, s);
+  };
+  // The ASM chain runs on activation records (the same outputs bit for bit), laid out above a
+  // caller's codes that may sit at the start of the workspace (the RMSNorm's) and followed by the
+  // tail tokens' codes; the other chains, and calls whose workspace cannot hold the records, on
+  // token-major codes.
+  const size_t base = x ? 0 : qbytes, tbytes = x && tail ? qa_bytes(tail, cols) : 0;
+  // (codes already quantized take one more launch to lay out, ~2.5 us, which the GEMM's gain of about
+  // 7 % covers from ~35 us on: 1.5e10 multiply-adds; Qwen3-8B QKV at 77 tokens, 1.9e9, lost 1.6 us)
+  long all_rows = 0;
+  for (int i = 0; i < n_mats; ++i) all_rows += rows[i];
+  const bool gains = x || opt(kGemmKind) == 1 || (double)main_n * cols * all_rows >= 1.5e10;
+  if (main_chain == KQ4_CHAIN_ASM && gains &&
+      rec_fits(ds, ws, n_mats, rows, cols, main_n, 0, pl, base + tbytes + pbytes, s)) {
+    Carve cv{static_cast<char *>(ws.b->p), base};
+    uint8_t *rec = cv.take<uint8_t>(kq4_rec_bytes(main_n, cols));
+    const int8_t *tq = nullptr;
+    const float *td = nullptr;
+    if (x) {
+      int8_t *q = tail ? cv.take<int8_t>((size_t)tail * cols) : nullptr;
+      float *d = tail ? cv.take<float>((size_t)tail * nb) : nullptr;
+      KQ4_HIP((hipError_t)kq4_launch_quantize_rec(x, xu, rec, q, d, main_n, n, cols, s));
+      tq = q;
+      td = d;
+    } else {
+      KQ4_HIP((hipError_t)kq4_launch_rec_from_q8(xq_in, xd_in, rec, main_n, cols, s));
+      tq = xq_in + (size_t)main_n * cols;
+      td = xd_in + (size_t)main_n * nb;
+    }
+    float *part = pbytes ? cv.take<float>(pbytes / sizeof(float)) : nullptr;
+    if ((rc = rec_gemms(n_mats, out, res, w, rows, cols, main_n, 0, rec, pl, part, s))) return rc;
+    return tail_gemv(tq, td);
   }
-  KQ4GemmPlan pl[KQ4_MAX_MATS];
-  const size_t pbytes = split_bytes(n_mats, rows, cols, main_n, 0, main_chain, ds->ncu, pl);
   if ((rc = ensure_ws(ws, qbytes + pbytes, s))) return rc;
   Carve cv{static_cast<char *>(ws.b->p)};
   KQ4GemmAct act;
@@ -494,7 +549,7 @@ int matmul_impl(int n_mats, float *const *out, const float *const *res, const ui
     // token rows per block at a stride, and the tail GEMV reads its rows as they are)
     int8_t *q = cv.take<int8_t>((size_t)n * cols);
     float *d = cv.take<float>((size_t)n * nb);
-    KQ4_HIP((hipError_t)kq4_launch_quantize(x, q, d, nullptr, n, cols, 0, s, 0, xu));
+    KQ4_HIP((hipError_t)kq4_launch_quantize(x, q, d, nullptr, n, cols, 0, s, xu));
     act = KQ4GemmAct{q, cols, 32, d, nb, 1};
     xq_t = q + (size_t)main_n * cols;
     xd_t = d + (size_t)main_n * nb;
@@ -509,17 +564,7 @@ int matmul_impl(int n_mats, float *const *out, const float *const *res, const ui
     KQ4_HIP((hipError_t)kq4_launch_gemm(out[i], res ? res[i] : nullptr, w[i], act, rows[i], cols,
                                         main_n, main_chain, ds->ncu, s, 0, pl[i].tile,
                                         pl[i].ksplit, part, opt(kGemmPrio)));
-  if (tail) {
-    float *o2[KQ4_MAX_MATS];
-    const float *r2[KQ4_MAX_MATS];
-    for (int i = 0; i < n_mats; ++i) {
-      o2[i] = out[i] + (size_t)main_n * rows[i];
-      r2[i] = (res && res[i]) ? res[i] + (size_t)main_n * rows[i] : nullptr;
-    }
-    return run_gemv(ds, ws, n_mats, o2, r2, w, rows, cols, nullptr, nullptr, xq_t, xd_t, tail, 0,
-                    s);
-  }
-  return KQ4_OK;
+  return tail_gemv(xq_t, xd_t);
 }
 
 // Workspace bytes of the expert FFN's staging (expert CSR, slot records, quantized X and av,
@@ -706,11 +751,11 @@ void kq4_shutdown(void) {
 
 size_t kq4_matmul_workspace_bytes(int n_batch, int cols) {
   if (n_batch < 0 || cols <= 0 || cols % 32) return 0;
-  // quantized activations (int8 or the fp8 GEMM's operand pairs) and the one-token RMSNorm row;
-  // beyond the GEMV's tokens the planner's K-split partial sums, at most KQ4_SPLIT_PART_MAX
-  const size_t q = qa_bytes(n_batch, cols), f = f8_bytes(n_batch, cols);
-  const size_t part = n_batch > KQ4_GEMV_MAX_M ? (size_t)KQ4_SPLIT_PART_MAX : 0;
-  return (q + part > f ? q + part : f) + al256((size_t)cols * sizeof(float));
+  // quantized activations and the one-token RMSNorm row; beyond the GEMV's tokens the prefill GEMM's
+  // activation records and the planner's K-split partial sums, at most KQ4_SPLIT_PART_MAX
+  size_t n = qa_bytes(n_batch, cols) + al256((size_t)cols * sizeof(float));
+  if (n_batch > KQ4_GEMV_MAX_M) n += al256(kq4_rec_bytes(n_batch, cols)) + (size_t)KQ4_SPLIT_PART_MAX;
+  return n;
 }
 
 size_t kq4_moe_workspace_bytes(int T, int tk, int ne, int d, int ef) {
@@ -801,7 +846,7 @@ int kq4_quantize_dev(int8_t *xq, float *xd, float *xde, const float *x, int n_ba
     return fail(KQ4_EINVAL, "quantize: x must be 16-byte, xq 8-byte aligned");
   KQ4_HIP((hipError_t)kq4_launch_quantize(x, xq, xd, xde, n_batch, cols,
                                           asm_tokens_for(chain, n_batch),
-                                          (hipStream_t)stream, 0));
+                                          (hipStream_t)stream));
   return KQ4_OK;
 }
 
@@ -910,13 +955,13 @@ int kq4_matmul_noalloc_dev(float *out, const float *x, const float *residual, co
   if (n_batch > 0 && cols > 0 && cols % 32 == 0) {
     if (n_batch <= KQ4_GEMV_MAX_M) {
       need = qa_bytes(n_batch, cols);
-    } else {   // fp8 operands, or int8 operands and the K-split partial sums
+    } else {   // token-major operands and the K-split partial sums, or the documented limit
       const int main_n = chain == KQ4_CHAIN_AUTO ? (n_batch & ~3) : n_batch;
       const int mc = chain == KQ4_CHAIN_AUTO ? KQ4_CHAIN_ASM : chain;
       KQ4GemmPlan pl;
       const size_t q = qa_bytes(n_batch, cols) + split_bytes(1, &rows, cols, main_n, 0, mc,
                                                              ds->ncu, &pl);
-      const size_t f = f8_bytes(n_batch, cols);
+      const size_t f = noalloc_bytes(n_batch, cols);
       need = q > f ? q : f;
     }
   }

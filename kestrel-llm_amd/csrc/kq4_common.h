@@ -121,6 +121,57 @@ KQ4_DEV float kq4_quad_bcast(float v, int m) {
   }
 }
 
+// Issue priority by progress through K (q8 = eighths done); see kq4_gemm.hip.
+KQ4_DEV void kq4_prio_by_progress(int q8) {
+  if (q8 < 4) __builtin_amdgcn_s_setprio(3);
+  else if (q8 < 6) __builtin_amdgcn_s_setprio(2);
+  else if (q8 < 7) __builtin_amdgcn_s_setprio(1);
+  else __builtin_amdgcn_s_setprio(0);
+}
+
+// 8 consecutive floats at x + off, or with `up` their silu_mul(x, up).
+KQ4_DEV void kq4_load8_silu(const float *__restrict__ x, const float *__restrict__ up, size_t off,
+                            float (&v)[8]) {
+  const float4 v0 = *reinterpret_cast<const float4 *>(x + off);
+  const float4 v1 = *reinterpret_cast<const float4 *>(x + off + 4);
+  v[0] = v0.x; v[1] = v0.y; v[2] = v0.z; v[3] = v0.w;
+  v[4] = v1.x; v[5] = v1.y; v[6] = v1.z; v[7] = v1.w;
+  if (up) {
+    const float4 u0 = *reinterpret_cast<const float4 *>(up + off);
+    const float4 u1 = *reinterpret_cast<const float4 *>(up + off + 4);
+    const float u[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = kq4_silu_mul(v[i], u[i]);
+  }
+}
+
+// A lane quad's 32-block (8 values per lane) quantized as quantize_row_q8_0_act does: the lane's 8
+// codes in pk, the block's scale returned. Each x/d is the Markstein-corrected quotient (see
+// kq4_quant.hip).
+KQ4_DEV float kq4_quantize8(const float (&v)[8], uint32_t (&pk)[2]) {
+  float a = 1e-10f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) a = fmaxf(a, fabsf(v[i]));
+  a = kq4_quad_max_pos(a);
+  const float d = a / 127.0f;
+  const float y = 1.0f / d;
+  int c[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    float q = v[i] * y;
+    const float e = fmaf(-q, d, v[i]);
+    q = fmaf(e, y, q);
+    c[i] = (int)(q + 0.5f);
+    c[i] = c[i] > 127 ? 127 : (c[i] < -127 ? -127 : c[i]);
+  }
+  // low bytes of c[0..3], c[4..7] into one dword each: two byte selects and an or
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    pk[k] = __builtin_amdgcn_perm((uint32_t)c[4 * k + 1], (uint32_t)c[4 * k], 0x0c0c0400u) |
+            __builtin_amdgcn_perm((uint32_t)c[4 * k + 3], (uint32_t)c[4 * k + 2], 0x04000c0cu);
+  return d;
+}
+
 // 16-byte load with the non-temporal hint (global_load_dwordx4 ... nt), for data read once per
 // launch (weight streams): measured on MI355X, plain streaming reads of 7-56 MB run 9-14 %
 // faster with it than without.
@@ -147,44 +198,6 @@ KQ4_DEV float kq4_max32(float v) {
 // 4 x int8 dot product accumulated into c (v_dot4_i32_i8).
 KQ4_DEV int kq4_dot4(uint32_t a, uint32_t b, int c) {
   return __builtin_amdgcn_sdot4((int)a, (int)b, c, false);
-}
-
-// ---- fp8 (OCP e4m3) operands of the prefill GEMM -------------------------------------------
-// The GEMM's matrix-core operands hold small integers exactly in e4m3 (sign, 4 exponent bits with
-// bias 7, 3 mantissa bits): weights w = n - 8 in [-8, 7]; activations q in [-127, 127] split as
-// q = 16*qh + ql with qh = q >> 4 in [-8, 7] and ql = q & 15 in [0, 15], entering as 16*qh and
-// ql. Every product and every partial sum of a block is an integer below 2^24, so the fp32
-// result of the fp8 MFMA is the exact block sum S.
-// e4m3 bytes of v = -8 .. 7 (index v + 8): the low 8 and the high 8 of the table.
-#define KQ4_E4M3_NEG 0xb8c0c4c8caccced0ull   // v = -8 .. -1
-#define KQ4_E4M3_POS 0x4e4c4a4844403800ull   // v =  0 ..  7
-
-// e4m3 byte of the integer v in [-8, 7].
-KQ4_DEV uint32_t kq4_e4m3_i4(int v) {
-  const uint64_t t = v < 0 ? KQ4_E4M3_NEG : KQ4_E4M3_POS;
-  return (uint32_t)(t >> (8 * (v & 7))) & 0xFFu;
-}
-
-// e4m3 bytes of 16*qh and ql for an int8 code q (16*qh is qh's e4m3 with the exponent 4 higher;
-// ql >= 8 lies in the binade [8, 16) whose step is 1: byte 0x48 + ql).
-KQ4_DEV uint32_t kq4_e4m3_hi(int q) {
-  const int qh = q >> 4;
-  return qh ? kq4_e4m3_i4(qh) + 0x20u : 0u;
-}
-KQ4_DEV uint32_t kq4_e4m3_lo(int q) {
-  const int ql = q & 15;
-  return ql < 8 ? kq4_e4m3_i4(ql) : 0x48u + (uint32_t)ql;
-}
-
-// The e4m3 bytes of the four 4-bit two's complement codes in the low nibbles of t's bytes (t's
-// high nibbles zero): a byte permute picks each from the table of its sign, a third one the
-// right table per byte.
-KQ4_DEV uint32_t kq4_e4m3_nib4(uint32_t t) {
-  const uint32_t pos = __builtin_amdgcn_perm((uint32_t)(KQ4_E4M3_POS >> 32), (uint32_t)KQ4_E4M3_POS, t);
-  const uint32_t neg = __builtin_amdgcn_perm((uint32_t)(KQ4_E4M3_NEG >> 32), (uint32_t)KQ4_E4M3_NEG,
-                                             t & 0x07070707u);
-  const uint32_t sel = ((t >> 1) & 0x04040404u) | 0x03020100u;   // byte k: k (pos) or 4 + k (neg)
-  return __builtin_amdgcn_perm(neg, pos, sel);
 }
 
 // ---- raw buffer loads -------------------------------------------------------------------------

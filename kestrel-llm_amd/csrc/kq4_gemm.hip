@@ -53,13 +53,6 @@ KQ4_DEV int kq4_mfma_tok(int v, int half) { return 8 * (v >> 2) + 4 * half + (v 
 // into 512 workgroups, 104 -> 98.5 us; down M = 2048, 512 workgroups, 330 -> 322 us; gate
 // M = 2048, three rounds, 291 -> 286 us). Results do not depend on it. The launcher turns it on
 // for 128 x 128 launches of whole rounds and for every pipelined 64 x 128 launch.
-KQ4_DEV void kq4_prio_by_progress(int q8) {
-  if (q8 < 4) __builtin_amdgcn_s_setprio(3);
-  else if (q8 < 6) __builtin_amdgcn_s_setprio(2);
-  else if (q8 < 7) __builtin_amdgcn_s_setprio(1);
-  else __builtin_amdgcn_s_setprio(0);
-}
-
 // TM / TN = MFMA token / row tiles per wave: a workgroup covers BM = 64*TM tokens x BN = 64*TN
 // rows (128 x 128, or smaller when the launch would otherwise have fewer than two tiles per CU).
 // Split K (ksplit > 1): the launch covers ksplit K slices of ks blocks (a multiple of the
@@ -596,246 +589,6 @@ __global__ __launch_bounds__(256, (TM == 2 && TN == 1) || (TM == 1 && TN == 2 &&
     }
 }
 
-// ---- fp8 formulation (ASM and GEMV32 chains over q4 weights) -----------------------------
-// The block sums come from v_mfma_f32_32x32x64_f8f6f4 on exactly representable integers (see
-// kq4_common.h): A = the activations' operand pairs [16*qh | ql] (64 e4m3 bytes per token and
-// block, written by the quantizer), B = [w | w] (the weights' 32 e4m3 bytes, read by both lane
-// halves), so the MFMA's fp32 result is S itself, exact; the scale products fl(wd * xs) of a
-// 32 x 32 tile come from v_mfma_f32_32x32x1_2b_f32 as outer products (one product per output,
-// rounded once: exactly the VALU's fl(wd * xs)); each output then takes one fma per block:
-// acc = fma(S, fl(wd * xs), acc), the same chain as the int8 kernel above, bit for bit. One
-// 32 x 32 tile per block costs 64 + 32 matrix-core cycles and 16 VALU fmas, against 32 and 48
-// (convert, product, fma) for the int8 form, so the VALU no longer bounds the kernel.
-// Stages of 2 blocks, double-buffered in LDS (one barrier per stage): activations 64 B per
-// (token, block) at an 80-B pitch, weights unpacked to e4m3 when stored (kq4_e4m3_nib4) at a
-// 48-B pitch, f32 row and token scales.
-#define KQ4_F8_KB 2
-#define KQ4_F8_AP 80
-#define KQ4_F8_BP 48
-
-typedef int kq4_v8i __attribute__((ext_vector_type(8)));
-KQ4_DEV kq4_v8i kq4_lds8(const uint8_t *p) {
-  const uint4 u0 = *reinterpret_cast<const uint4 *>(p);
-  const uint4 u1 = *reinterpret_cast<const uint4 *>(p + 16);
-  return kq4_v8i{(int)u0.x, (int)u0.y, (int)u0.z, (int)u0.w,
-                 (int)u1.x, (int)u1.y, (int)u1.z, (int)u1.w};
-}
-
-template <int CHAIN, int TM, int TN>
-__global__ __launch_bounds__(256, 2) void kq4_gemm_f8_kernel(
-    float *__restrict__ out, const float *__restrict__ res, const uint8_t *__restrict__ w,
-    const uint8_t *__restrict__ xp, const float *__restrict__ xd, int rows, int n_tok, int nb,
-    int nst, int mtiles, int ntiles, long wbytes) {
-  constexpr int BM = 64 * TM, BN = 64 * TN;
-  constexpr int NA = BM / 32;   // 16-B activation pieces per thread and stage
-  __shared__ __align__(16) uint8_t sA[2][KQ4_F8_KB][BM * KQ4_F8_AP];
-  __shared__ __align__(16) uint8_t sB[2][KQ4_F8_KB][BN * KQ4_F8_BP];
-  __shared__ __align__(16) float sX[2][KQ4_F8_KB][BM];
-  __shared__ __align__(16) float sW[2][KQ4_F8_KB][BN];
-
-  // XCD-aware tile order, as the int8 kernel
-  const int ntile = mtiles * ntiles;
-  const int wg = blockIdx.x;
-  const int xcd = wg & 7, q8 = ntile >> 3, r8 = ntile & 7;
-  const int tile = xcd * q8 + (xcd < r8 ? xcd : r8) + (wg >> 3);
-  const int m0 = (tile % mtiles) * BM;
-  const int n0 = (tile / mtiles) * BN;
-  const int t = threadIdx.x;
-  const int lane = t & 63;
-  const int wave = t >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int l32 = lane & 31, half = lane >> 5;
-
-  float acc[TM][TN][16];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-
-  struct Regs {
-    uint4 a[NA];
-    uint4 b;
-    uint32_t sw;
-    float x0, x1;
-  };
-  // global -> registers for the stage at block b0 (even): activation pieces (token idx >> 3,
-  // block (idx >> 2) & 1, 16-B piece idx & 3); one stream-layout unit per thread of the first
-  // 2 * BN (row set t >> 6, lane t & 63: the half-row of blocks b0 and b0 + 1); row scales (the
-  // two f16 of blocks b0, b0 + 1, adjacent) for t < BN, token scales for t in [128, 128 + BM)
-  // Buffer loads (kq4_rsrc): tokens past n_tok, rows past the matrix and the block past an odd
-  // nb read zeros without branches.
-  const __amdgpu_buffer_rsrc_t ra = kq4_rsrc(xp, (uint32_t)((size_t)n_tok * nb * 64));
-  const __amdgpu_buffer_rsrc_t rw = kq4_rsrc(w, (uint32_t)wbytes);
-  const __amdgpu_buffer_rsrc_t rx = kq4_rsrc(xd, (uint32_t)((size_t)n_tok * nb * 4));
-  auto load = [&](Regs &rg, int b0) {
-#pragma unroll
-    for (int u = 0; u < NA; ++u) {
-      const int idx = t + 256 * u;
-      const int tok = idx >> 3, bl = (idx >> 2) & 1, pc = idx & 3;
-      const uint32_t off =
-          b0 + bl < nb ? ((uint32_t)(m0 + tok) * nb + b0 + bl) * 64u + 16u * pc : KQ4_OOB;
-      rg.a[u] = kq4_bload16(ra, off);
-    }
-    rg.b = kq4_bload16(rw, t < 2 * BN ? (uint32_t)kq4_stream_nib(n0 + 32 * (t >> 6) + (lane & 31),
-                                                                  b0, lane >> 5, nst)
-                                       : KQ4_OOB);
-    rg.sw = kq4_bload4(rw, t < BN ? (uint32_t)kq4_stream_scale(n0 + t, b0, nst) : KQ4_OOB);
-    const int tok = t - 128;
-    const uint32_t xo = ((uint32_t)(m0 + tok) * nb + b0) * 4u;
-    const bool xt = t >= 128 && t < 128 + BM;
-    rg.x0 = __uint_as_float(kq4_bload4(rx, xt ? xo : KQ4_OOB));
-    rg.x1 = __uint_as_float(kq4_bload4(rx, xt && b0 + 1 < nb ? xo + 4 : KQ4_OOB));
-  };
-  auto store = [&](const Regs &rg, int buf) {
-#pragma unroll
-    for (int u = 0; u < NA; ++u) {
-      const int idx = t + 256 * u;
-      const int tok = idx >> 3, bl = (idx >> 2) & 1, pc = idx & 3;
-      *reinterpret_cast<uint4 *>(&sA[buf][bl][tok * KQ4_F8_AP + 16 * pc]) = rg.a[u];
-    }
-    if (t < 2 * BN) {
-      const int row = 32 * (t >> 6) + (lane & 31), h = lane >> 5;
-      // dword d of a block's half-row: low nibbles = elements 8d .. 8d+3, high = 8d+4 .. 8d+7
-      const uint32_t d[4] = {rg.b.x, rg.b.y, rg.b.z, rg.b.w};
-#pragma unroll
-      for (int bl = 0; bl < 2; ++bl) {
-        uint4 o;
-        o.x = kq4_e4m3_nib4(d[2 * bl] & 0x0F0F0F0Fu);
-        o.y = kq4_e4m3_nib4((d[2 * bl] >> 4) & 0x0F0F0F0Fu);
-        o.z = kq4_e4m3_nib4(d[2 * bl + 1] & 0x0F0F0F0Fu);
-        o.w = kq4_e4m3_nib4((d[2 * bl + 1] >> 4) & 0x0F0F0F0Fu);
-        *reinterpret_cast<uint4 *>(&sB[buf][bl][row * KQ4_F8_BP + 16 * h]) = o;
-      }
-    }
-    if (t < BN) {
-      sW[buf][0][t] = kq4_h2f(rg.sw);
-      sW[buf][1][t] = kq4_h2f(rg.sw >> 16);
-    } else if (t >= 128 && t < 128 + BM) {
-      // ASM chain: the reference multiplies by the f16-rounded activation scale
-      sX[buf][0][t - 128] = CHAIN == KQ4_CHAIN_ASM ? kq4_f16_round(rg.x0) : rg.x0;
-      sX[buf][1][t - 128] = CHAIN == KQ4_CHAIN_ASM ? kq4_f16_round(rg.x1) : rg.x1;
-    }
-  };
-  auto compute = [&](int buf, int b0) {
-#pragma unroll
-    for (int bl = 0; bl < KQ4_F8_KB; ++bl) {
-      if (b0 + bl >= nb) break;
-      kq4_v8i a[TM], bq[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-        a[i] = kq4_lds8(&sA[buf][bl][(32 * TM * wm + 32 * i + l32) * KQ4_F8_AP + 32 * half]);
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-        bq[j] = kq4_lds8(&sB[buf][bl][(32 * TN * wn + 32 * j + l32) * KQ4_F8_BP]);
-      const kq4_v32f z32 = {0};
-      const kq4_v16f z16 = {0};
-      if constexpr (TM == 2) {
-        // the outer product's two blocks are the wave's two token tiles (lanes 0-31, 32-63)
-        const float xv = sX[buf][bl][64 * wm + lane];
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const float wv = sW[buf][bl][32 * TN * wn + 32 * j + l32];
-          const kq4_v32f c = __builtin_amdgcn_mfma_f32_32x32x1f32(xv, wv, z32, 0, 0, 0);
-#pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            const kq4_v16f sb =
-                __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[i], bq[j], z16, 0, 0, 0, 0, 0, 0);
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = fmaf(sb[v], c[16 * i + v], acc[i][j][v]);
-          }
-        }
-      } else {
-        // one token tile: the outer product's two blocks are the wave's row tiles
-        const float xv = sX[buf][bl][32 * wm + l32];
-        const float wv = sW[buf][bl][32 * TN * wn + (TN == 2 ? lane : l32)];
-        const kq4_v32f c = __builtin_amdgcn_mfma_f32_32x32x1f32(xv, wv, z32, 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const kq4_v16f sb =
-              __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[0], bq[j], z16, 0, 0, 0, 0, 0, 0);
-#pragma unroll
-          for (int v = 0; v < 16; ++v) acc[0][j][v] = fmaf(sb[v], c[16 * j + v], acc[0][j][v]);
-        }
-      }
-    }
-  };
-
-  Regs rg;
-  load(rg, 0);
-  store(rg, 0);
-  __syncthreads();
-  int buf = 0;
-  for (int b0 = 0; b0 < nb; b0 += KQ4_F8_KB) {
-    const bool more = b0 + KQ4_F8_KB < nb;
-    if (more) load(rg, b0 + KQ4_F8_KB);   // in flight during the compute
-    compute(buf, b0);
-    if (more) store(rg, buf ^ 1);         // the other buffer: nobody reads it this stage
-    __syncthreads();
-    buf ^= 1;
-  }
-
-  // out = [res +] acc
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int row = n0 + 32 * TN * wn + 32 * j + l32;
-      if (row >= rows) continue;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int tok = m0 + 32 * TM * wm + 32 * i + kq4_mfma_tok(v, half);
-        if (tok >= n_tok) continue;
-        const size_t o = (size_t)tok * rows + row;
-        out[o] = res ? res[o] + acc[i][j][v] : acc[i][j][v];
-      }
-    }
-}
-
-template <int TM, int TN>
-static hipError_t gemm_f8_launch(float *out, const float *res, const uint8_t *w, const uint8_t *xp,
-                                 const float *xd, int rows, int n_tok, int nb, int nst, int chain,
-                                 hipStream_t s) {
-  const int mtiles = (n_tok + 64 * TM - 1) / (64 * TM);
-  const int ntiles = (rows + 64 * TN - 1) / (64 * TN);
-  const dim3 grid((unsigned)(mtiles * ntiles));
-  const long wbytes = (long)kq4_stream_bytes(rows, nb * 32);
-  if (chain == KQ4_CHAIN_ASM)
-    hipLaunchKernelGGL((kq4_gemm_f8_kernel<KQ4_CHAIN_ASM, TM, TN>), grid, dim3(256), 0, s, out, res,
-                       w, xp, xd, rows, n_tok, nb, nst, mtiles, ntiles, wbytes);
-  else if (chain == KQ4_CHAIN_GEMV32)
-    hipLaunchKernelGGL((kq4_gemm_f8_kernel<KQ4_CHAIN_GEMV32, TM, TN>), grid, dim3(256), 0, s, out,
-                       res, w, xp, xd, rows, n_tok, nb, nst, mtiles, ntiles, wbytes);
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
-}
-
-int kq4_launch_gemm_f8(float *out, const float *res, const uint8_t *w, const uint8_t *xp,
-                       const float *xd, int rows, int cols, int n_tok, int chain, int ncu,
-                       hipStream_t s, int tile) {
-  const int nb = cols / 32;
-  const int nst = (nb + KQ4_STREAM_CB - 1) / KQ4_STREAM_CB;
-  if (n_tok <= 0 || rows <= 0) return 0;
-  if (chain != KQ4_CHAIN_ASM && chain != KQ4_CHAIN_GEMV32) return (int)hipErrorInvalidValue;
-  // 32-bit buffer offsets: operand pairs and weights below 4 GB
-  if (((size_t)n_tok + 128) * nb * 64 >= KQ4_OOB || kq4_stream_bytes(rows, cols) >= KQ4_OOB)
-    return (int)hipErrorInvalidValue;
-  auto tiles = [&](int bm, int bn) {
-    return (long)((n_tok + bm - 1) / bm) * ((rows + bn - 1) / bn);
-  };
-  // tile: 1 / 2 / 3 / 4 = 128x128 / 64x128 / 64x64 / 128x64 (tokens x rows), as the int8 form
-  const int pick = tile >= 1 && tile <= 4 ? tile
-                   : tiles(128, 128) >= 2L * ncu ? 1 : (tiles(64, 128) >= 2L * ncu ? 2 : 3);
-  hipError_t e;
-  if (pick == 1) e = gemm_f8_launch<2, 2>(out, res, w, xp, xd, rows, n_tok, nb, nst, chain, s);
-  else if (pick == 2) e = gemm_f8_launch<1, 2>(out, res, w, xp, xd, rows, n_tok, nb, nst, chain, s);
-  else if (pick == 4) e = gemm_f8_launch<2, 1>(out, res, w, xp, xd, rows, n_tok, nb, nst, chain, s);
-  else e = gemm_f8_launch<1, 1>(out, res, w, xp, xd, rows, n_tok, nb, nst, chain, s);
-  return (int)e;
-}
-
 // out[i] = [res[i] +] (..((out[i] + part[0][i]) + part[1][i]) .. + part[np-1][i]): the K
 // slices' outputs added in slice order, 4 floats per thread (n4 = elements / 4).
 __global__ __launch_bounds__(256) void kq4_split_reduce_kernel(float *__restrict__ out,
@@ -860,6 +613,14 @@ __global__ __launch_bounds__(256) void kq4_split_reduce_kernel(float *__restrict
     v.w = r.w + v.w;
   }
   reinterpret_cast<float4 *>(out)[i] = v;
+}
+
+int kq4_launch_split_reduce(float *out, const float *res, const float *part, int np, long pstride,
+                            hipStream_t s) {
+  const long n4 = pstride / 4;   // rows % 4 == 0
+  hipLaunchKernelGGL(kq4_split_reduce_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s,
+                     out, res, part, np, pstride, n4);
+  return (int)hipGetLastError();
 }
 
 template <int TM, int TN>
@@ -903,7 +664,7 @@ static hipError_t gemm_launch(float *out, const float *res, const uint8_t *w,
 
 // Blocks per K slice for ksplit slices: ceil(nb / ksplit) rounded up to whole stream-layout
 // stages; 0 when ksplit slices of that length do not all hold blocks.
-static int split_len(int nb, int cb, int ksplit) {
+int kq4_split_len(int nb, int cb, int ksplit) {
   if (ksplit < 2) return nb;
   const int ks = ((nb + ksplit - 1) / ksplit + cb - 1) / cb * cb;
   return (long)(ksplit - 1) * ks < nb ? ks : 0;
@@ -954,7 +715,7 @@ KQ4GemmPlan kq4_gemm_plan(int n_tok, int rows, int cols, int wf, int chain, int 
   // workspace's KQ4_SPLIT_PART_MAX
   auto most = [&](long t, long cap, int minb) {
     for (int k = KQ4_GEMM_SPLIT_MAX; k >= 2; --k)
-      if (k * t <= cap && split_len(nb, cb, k) >= minb &&
+      if (k * t <= cap && kq4_split_len(nb, cb, k) >= minb &&
           (long)(k - 1) * n_tok * rows * 4 <= (long)KQ4_SPLIT_PART_MAX)
         return k;
     return 1;
@@ -969,7 +730,7 @@ KQ4GemmPlan kq4_gemm_plan(int n_tok, int rows, int cols, int wf, int chain, int 
                                                       : 1;
   // forced slices: 0 / 1 none; counts the blocks do not allow are taken as none
   int fk = force_split;
-  if (fk >= 0 && (fk <= 1 || fk > KQ4_GEMM_SPLIT_MAX || !split_len(nb, cb, fk))) fk = 1;
+  if (fk >= 0 && (fk <= 1 || fk > KQ4_GEMM_SPLIT_MAX || !kq4_split_len(nb, cb, fk))) fk = 1;
   if (force_tile >= 1 && force_tile <= 4) {
     p.tile = force_tile;
     p.ksplit = fk >= 1 ? fk : force_tile == 1 ? ka : force_tile == tb ? kb : 1;
@@ -1002,7 +763,7 @@ int kq4_launch_gemm(float *out, const float *res, const uint8_t *w, const KQ4Gem
   auto tiles = [&](int bm, int bn) {
     return (long)((n_tok + bm - 1) / bm) * ((rows + bn - 1) / bn);
   };
-  const int ks = split_len(nb, cb, ksplit);
+  const int ks = kq4_split_len(nb, cb, ksplit);
   if (ksplit < 1 || ksplit > KQ4_GEMM_SPLIT_MAX || !ks || (ksplit > 1 && !part))
     return (int)hipErrorInvalidValue;
   int pick = tile >= 1 && tile <= 4 ? tile
@@ -1047,8 +808,5 @@ int kq4_launch_gemm(float *out, const float *res, const uint8_t *w, const KQ4Gem
     e = gemm_launch<1, 1>(out, ksplit > 1 ? nullptr : res, w, act, rows, n_tok, nb, nst, chain,
                           wf, wbytes, s, ksplit, ks, part, ps);
   if (e != hipSuccess || ksplit < 2) return (int)e;
-  const long n4 = ps / 4;   // rows % 4 == 0
-  hipLaunchKernelGGL(kq4_split_reduce_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s,
-                     out, res, part, ksplit - 1, ps, n4);
-  return (int)hipGetLastError();
+  return kq4_launch_split_reduce(out, res, part, ksplit - 1, ps, s);
 }

@@ -62,8 +62,7 @@ struct KQ4GemvArgs {
 
 // up != nullptr: quantizes silu_mul(x, up) instead of x (the dense FFN's down input).
 int kq4_launch_quantize(const float *x, int8_t *xq, float *xd, float *xde, int n_batch, int cols,
-                        int asm_tokens, hipStream_t stream, int block_major = 0,
-                        const float *up = nullptr);
+                        int asm_tokens, hipStream_t stream, const float *up = nullptr);
 // g[i] = silu_mul(g[i], u[i]) in place, the reference worker's element rule (g, u 16-B aligned).
 int kq4_launch_silu_mul(float *g, const float *u, long n, hipStream_t stream);
 // RMSNorm of n_batch rows of d (d % 8 == 0, d <= 16384; 16-B aligned rows), serial = 0 the chunked order of
@@ -120,12 +119,28 @@ int kq4_launch_gemm(float *out, const float *res, const uint8_t *w, const KQ4Gem
                     int wf = 0, int tile = 0, int ksplit = 1, float *part = nullptr,
                     int prio = -1);
 
-// Prefill GEMM on fp8 matrix-core operands (ASM or GEMV32 chain, q4 weights, bit-identical to
-// kq4_launch_gemm): xp = the activations' e4m3 operand pairs [n_tok][cols/32][64] (the
-// quantizer's block_major = 2 output), xd their f32 scales [n_tok][cols/32].
-int kq4_launch_gemm_f8(float *out, const float *res, const uint8_t *w, const uint8_t *xp,
-                       const float *xd, int rows, int cols, int n_tok, int chain, int ncu,
-                       hipStream_t stream, int tile = 0);
+// Blocks per K slice for ksplit slices (whole stream-layout stages of cb blocks); 0 when they do
+// not all hold blocks. The slices' outputs added in slice order, then the residual.
+int kq4_split_len(int nb, int cb, int ksplit);
+int kq4_launch_split_reduce(float *out, const float *res, const float *part, int np, long pstride,
+                            hipStream_t s);
+
+// Prefill GEMM of the ASM chain (q4) and the Q8GEMM chain (wf = 1) on activation records
+// (kq4_gemm_rec.hip), bit-identical to kq4_launch_gemm at the same ksplit. rec: kq4_rec_bytes(n_tok,
+// cols) bytes made by kq4_launch_quantize_rec (tokens [n_main, n) as int8 codes xq / scales xd,
+// token-major, for the decode GEMV) or kq4_launch_rec_from_q8.
+size_t kq4_rec_bytes(int n, int cols);
+int kq4_launch_quantize_rec(const float *x, const float *up, uint8_t *rec, int8_t *xq, float *xd,
+                            int n_main, int n, int cols, hipStream_t s);
+int kq4_launch_rec_from_q8(const int8_t *xq, const float *xd, uint8_t *rec, int n, int cols,
+                           hipStream_t s);
+int kq4_gemm_rec_ok(int rows, int cols, int n_tok, int wf);   // within 32-bit buffer offsets
+// The record form's tile for a launch the planner runs as `plan` (its K slices are kept), or 0 where
+// the token-major form is faster.
+int kq4_rec_tile(int n_tok, int rows, int wf, int ncu, const KQ4GemmPlan &plan);
+int kq4_launch_gemm_rec(float *out, const float *res, const uint8_t *w, const uint8_t *rec, int rows,
+                        int cols, int n_tok, int wf, hipStream_t s, int tile, int ksplit,
+                        float *part, int prio);
 
 // MoE
 int kq4_launch_moe_route(int *sel, float *pr, const float *logits, int T, int ne, int tk,

@@ -18,100 +18,39 @@
 // significands (all 2^46, kestrel-llm_amd/probe/kq4_div_probe.hip), hence for all operands here
 // whose residual stays normal; where it would not (|x| < 2^-102, while d >= 1e-10/127), |x/d| is
 // below 2^-61 and both give code 0.
-// Token-major output: a wave's 16 quads take 16 consecutive blocks of a token. Block-major
-// output ([b][m][32]): a wave's 16 quads take 4 tokens x 4 blocks, so each block's 128 B of
-// codes for the 4 tokens is written whole by one store instruction (one quad per block in
-// token-major order would leave each 128-B line to four workgroups, on different XCDs).
+// A wave's 16 quads take 16 consecutive blocks of a token. (The prefill GEMM's records are written by
+// kq4_quantize_rec_kernel, kq4_gemm_rec.hip.)
 __global__ __launch_bounds__(256) void kq4_quantize_kernel(const float *__restrict__ x,
                                                            const float *__restrict__ up,
                                                            int8_t *__restrict__ xq,
                                                            float *__restrict__ xd,
                                                            float *__restrict__ xde, int n_batch,
-                                                           int cols, int nb, int asm_tokens,
-                                                           int block_major) {
+                                                           int cols, int nb, int asm_tokens) {
   const int qq = threadIdx.x & 3;
   const long gq = (long)blockIdx.x * (blockDim.x >> 2) + (threadIdx.x >> 2);
-  int m, b;
-  if (block_major == 1) {
-    const long g = gq >> 4;
-    const int qi = (int)(gq & 15), nbg = (nb + 3) >> 2;
-    m = (int)(g / nbg) * 4 + (qi & 3);
-    b = (int)(g % nbg) * 4 + (qi >> 2);
-    if (m >= n_batch || b >= nb) return;   // whole quads exit together
-  } else {
-    if (gq >= (long)n_batch * nb) return;
-    m = (int)(gq / nb);
-    b = (int)(gq - (long)m * nb);
-  }
-  const long blk = (long)m * nb + b;
+  if (gq >= (long)n_batch * nb) return;
+  const int m = (int)(gq / nb), b = (int)(gq - (long)m * nb);
   const size_t off = (size_t)m * cols + (size_t)b * 32 + 8 * qq;
-  const float4 v0 = *reinterpret_cast<const float4 *>(x + off);
-  const float4 v1 = *reinterpret_cast<const float4 *>(x + off + 4);
-  float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-  if (up) {
-    const float4 u0 = *reinterpret_cast<const float4 *>(up + off);
-    const float4 u1 = *reinterpret_cast<const float4 *>(up + off + 4);
-    const float u[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = kq4_silu_mul(v[i], u[i]);
-  }
-  float a = 1e-10f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) a = fmaxf(a, fabsf(v[i]));
-  a = kq4_quad_max_pos(a);
-  const float d = a / 127.0f;
-  const float y = 1.0f / d;
-  int c[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    float q = v[i] * y;
-    const float e = fmaf(-q, d, v[i]);
-    q = fmaf(e, y, q);
-    c[i] = (int)(q + 0.5f);
-    c[i] = c[i] > 127 ? 127 : (c[i] < -127 ? -127 : c[i]);
-  }
-  // low bytes of c[0..3], c[4..7] into one dword each: two byte selects and an or
+  float v[8];
+  kq4_load8_silu(x, up, off, v);
   uint32_t pk[2];
-#pragma unroll
-  for (int k = 0; k < 2; ++k)
-    pk[k] = __builtin_amdgcn_perm((uint32_t)c[4 * k + 1], (uint32_t)c[4 * k], 0x0c0c0400u) |
-            __builtin_amdgcn_perm((uint32_t)c[4 * k + 3], (uint32_t)c[4 * k + 2], 0x04000c0cu);
-  // token-major [m][cols] / [m][nb], block-major [b][m][32] / [b][m], or (block_major = 2) the
-  // fp8 GEMM's operand pairs [m][nb][64]: the e4m3 bytes of 16*(q >> 4) for the block's 32
-  // elements, then those of q & 15 (kq4_e4m3_hi / _lo), scales token-major
-  const size_t so = block_major == 1 ? (size_t)b * n_batch + m : (size_t)blk;
-  if (block_major == 2) {
-    uint32_t hi[2] = {0, 0}, lo[2] = {0, 0};
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int q = (int)(int8_t)(pk[i >> 2] >> (8 * (i & 3)));
-      hi[i >> 2] |= kq4_e4m3_hi(q) << (8 * (i & 3));
-      lo[i >> 2] |= kq4_e4m3_lo(q) << (8 * (i & 3));
-    }
-    uint8_t *pair = reinterpret_cast<uint8_t *>(xq) + (size_t)blk * 64 + 8 * qq;
-    *reinterpret_cast<uint2 *>(pair) = make_uint2(hi[0], hi[1]);
-    *reinterpret_cast<uint2 *>(pair + 32) = make_uint2(lo[0], lo[1]);
-  } else {
-    const size_t qo = block_major ? ((size_t)b * n_batch + m) * 32 + 8 * qq : off;
-    *reinterpret_cast<uint2 *>(xq + qo) = make_uint2(pk[0], pk[1]);
-  }
+  const float d = kq4_quantize8(v, pk);
+  *reinterpret_cast<uint2 *>(xq + off) = make_uint2(pk[0], pk[1]);
   if (qq == 0) {
-    xd[so] = d;
-    if (xde) xde[so] = (m < asm_tokens) ? kq4_f16_round(d) : d;
+    xd[gq] = d;
+    if (xde) xde[gq] = (m < asm_tokens) ? kq4_f16_round(d) : d;
   }
 }
 
 int kq4_launch_quantize(const float *x, int8_t *xq, float *xd, float *xde, int n_batch, int cols,
-                        int asm_tokens, hipStream_t stream, int block_major, const float *up) {
+                        int asm_tokens, hipStream_t stream, const float *up) {
   const int nb = cols / 32;
   const long nblk = (long)n_batch * nb;
   if (nblk <= 0) return 0;
   const int per_wg = 256 / 4;
-  // block-major: whole groups of 4 tokens x 4 blocks
-  const long quads = block_major == 1 ? (long)((n_batch + 3) / 4) * ((nb + 3) / 4) * 16 : nblk;
-  const long grid = (quads + per_wg - 1) / per_wg;
+  const long grid = (nblk + per_wg - 1) / per_wg;
   hipLaunchKernelGGL(kq4_quantize_kernel, dim3((unsigned)grid), dim3(256), 0, stream, x, up, xq, xd,
-                     xde, n_batch, cols, nb, asm_tokens, block_major);
+                     xde, n_batch, cols, nb, asm_tokens);
   return (int)hipGetLastError();
 }
 

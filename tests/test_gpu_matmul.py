@@ -209,6 +209,38 @@ def test_gemm_tile_forms_bit_exact(kq4, torch_dev, orc, tile, chain, kind):
     assert np.array_equal(got[tok, row].view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("q8", [False, True])
+@pytest.mark.parametrize("n,rows,cols,tile,split", [
+    (17, 4, 32, 3, 1), (64, 36, 64, 2, 1), (65, 132, 96, 1, 1), (127, 260, 480, 1, 1),
+    (129, 128, 544, 2, 1), (200, 100, 1056, 3, 1), (300, 264, 2080, 1, 2), (190, 392, 2592, 2, 4)])
+def test_gemm_records_match_token_major(kq4, torch_dev, q8, n, rows, cols, tile, split):
+    """The record form of the prefill GEMM (gemm_kind = 1) gives the token-major form's bits at the
+    edges of its token groups, row sets, stages (odd block counts: a stage past K) and K slices, with
+    a tail, a residual and, for q4, activations already quantized."""
+    torch = torch_dev
+    x = to_dev(torch, synth.make_activations(n, cols, n + cols))
+    res = to_dev(torch, synth.make_activations(n, rows, n + 1))
+    if q8:
+        w = kq4.q8_prepare_dev(synth.make_q8_weights(rows, cols, rows, g=4), rows, cols, g=4)
+    else:
+        w = wdev(kq4, torch, synth.make_q4_weights(rows, cols, rows), rows, cols)
+        xq = torch.empty((n, cols), dtype=torch.int8, device="cuda")
+        xd = torch.empty((n, cols // 32), dtype=torch.float32, device="cuda")
+        kq4.quantize_dev(x, xq, xd)
+    outs = []
+    for kind in (0, 1):
+        with kq4.options(gemm_kind=kind, gemm_tile=tile, gemm_split=split):
+            o = torch.full((n, rows), float("nan"), dtype=torch.float32, device="cuda")
+            (kq4.q8_matmul_dev if q8 else kq4.matmul_dev)(o, x, w, rows, cols, residual=res)
+            outs.append(host(o))
+            if not q8:
+                kq4.matmul_q_dev(o, xq, xd, w, rows, cols, n, residual=res)
+                outs.append(host(o))
+    torch.cuda.synchronize()
+    for o in outs[1:]:
+        assert np.array_equal(o.view(np.uint32), outs[0].view(np.uint32))
+
+
 @pytest.mark.parametrize("form", ["matmul", "silu", "multi"])
 def test_gemm_f8_auto_tail(kq4, torch_dev, orc, form):
     """The fp8-operand GEMM (gemm_kind = 1) with an AUTO-chain tail: 301 tokens are 300 on fp8
