@@ -572,7 +572,8 @@ int matmul_impl(int n_mats, float *const *out, const float *const *res, const ui
 size_t moe_stage_bytes(int T, int tk, int ne, int d, int ef) {
   const size_t np = (size_t)T * tk;
   return al256((ne + 1) * sizeof(int)) + al256(np * sizeof(int)) +
-         al256((size_t)ne * KQ4_MOE_REC * sizeof(int)) + al256((size_t)T * d) +
+         al256((size_t)ne * KQ4_MOE_REC * sizeof(int)) +
+         al256((1 + 4 * (np / 32 + ne)) * sizeof(int)) + al256((size_t)T * d) +
          al256((size_t)T * (d / 32) * sizeof(float)) + al256(np * ef) +
          al256(np * (ef / 32) * sizeof(float)) + al256(np * d * sizeof(float));
 }
@@ -605,6 +606,7 @@ int moe_impl(float *Y, const float *X, const int *sel, const float *pr, int T, i
   ws.ex_off = cv.take<int>(ne + 1);
   ws.ex_pair = cv.take<int>(np);
   ws.rec = cv.take<int>((size_t)ne * KQ4_MOE_REC);
+  ws.tiles = cv.take<int>(1 + 4 * (np / 32 + ne));
   ws.xq = cv.take<int8_t>((size_t)T * d);
   ws.xd = cv.take<float>((size_t)T * (d / 32));
   ws.avq = cv.take<int8_t>(np * ef);

@@ -156,6 +156,7 @@ struct KQ4MoeWs {
   int *ex_pair;  // [T*tk] (t*tk+j) grouped by expert
   int *rec;      // [ne][KQ4_MOE_REC] slot records (active experts in id order): expert (-1 past
                  // them), offset of its pairs in ex_pair, pair count, its first pair ids
+  int *tiles;    // [1 + 4*(T*tk/32 + ne)] grouped-GEMM tiles: count, then expert, offset, pairs, 0
   int8_t *xq;    // [T][d]
   float *xd;     // [T][d/32]
   int8_t *avq;   // [T*tk][ef]
@@ -163,6 +164,12 @@ struct KQ4MoeWs {
   float *P;      // [T*tk][d]
   int ncu;       // compute units of the device (sizes the down projection's workgroups)
 };
+// The expert projections as a grouped GEMM over 32-pair tiles (kq4_moe_gemm.hip): whether a launch takes
+// it, and the gate/up (down = 0: G, U) or down (down = 1: D, D) launch.
+int kq4_moe_gemm_ok(int T, int tk, int ne, int d, int ef);
+int kq4_launch_moe_gemm(int down, const uint8_t *w0, const uint8_t *w1, const KQ4MoeWs &ws, int T,
+                        int tk, int ne, int d, int ef, float *g_out, float *u_out, float *av_out,
+                        hipStream_t s);
 // Shapes the MoE kernels take: d, ef multiples of 32, d <= 4096, ef <= 3840.
 int kq4_moe_shape_ok(int d, int ef);
 int kq4_launch_moe_dbg(float *Y, const float *X, const int *sel, const float *pr, int T, int tk,

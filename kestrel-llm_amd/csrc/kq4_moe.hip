@@ -310,7 +310,8 @@ int kq4_launch_moe_logits(float *logits, const float *router, const float *X, in
 // expert workgroup finds its expert and pairs with one load instead of a chain of three.
 // Workgroups 1..: the activation quantizer of kq4_quant.hip (one half-wave per 32-block).
 __global__ __launch_bounds__(256) void kq4_moe_prep_kernel(
-    int *__restrict__ ex_off, int *__restrict__ ex_pair, int *__restrict__ rec, int nslot,
+    int *__restrict__ ex_off, int *__restrict__ ex_pair, int *__restrict__ rec,
+    int *__restrict__ tiles, int nslot,
     const int *__restrict__ sel, int n_pairs, int ne, const float *__restrict__ X,
     int8_t *__restrict__ xq, float *__restrict__ xd, int T, int d) {
   if (blockIdx.x == 0) {
@@ -329,9 +330,13 @@ __global__ __launch_bounds__(256) void kq4_moe_prep_kernel(
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       if (ev[j] >= 0 && ev[j] < ne) atomicAdd(&cnt[ev[j]], 1);
-    for (int i = tid + 4 * nt; i < n_pairs; i += nt) {
-      const int e = sel[i];
-      if (e >= 0 && e < ne) atomicAdd(&cnt[e], 1);
+    for (int i0 = tid + 4 * nt; i0 < n_pairs; i0 += 8 * nt) {   // (8 loads in flight per thread)
+      int v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = i0 + nt * j < n_pairs ? sel[i0 + nt * j] : -1;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (v[j] >= 0 && v[j] < ne) atomicAdd(&cnt[v[j]], 1);
     }
     __syncthreads();
     // exclusive scans of the counts and of the active flags: thread tid owns experts
@@ -339,22 +344,27 @@ __global__ __launch_bounds__(256) void kq4_moe_prep_kernel(
     // waves' totals (through LDS, one barrier) give each wave its offset and every thread the
     // block totals tc (pairs) and ta (active experts).
     const int per = (ne + nt - 1) / nt, e0 = tid * per;
-    int sc = 0, sa = 0;
-    for (int e = e0; e < e0 + per && e < ne; ++e) { sc += cnt[e]; sa += cnt[e] > 0; }
+    int sc = 0, sa = 0, sg = 0;   // pairs, active experts, 32-pair tiles
+    for (int e = e0; e < e0 + per && e < ne; ++e) {
+      sc += cnt[e];
+      sa += cnt[e] > 0;
+      sg += (cnt[e] + 31) >> 5;
+    }
     const int lane = tid & 63, wv = tid >> 6, nwv = nt >> 6;
-    int ic = sc, ia = sa;   // inclusive scans within the wave
+    int ic = sc, ia = sa, ig = sg;   // inclusive scans within the wave
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-      const int vc = __shfl_up(ic, o, 64), va = __shfl_up(ia, o, 64);
-      if (lane >= o) { ic += vc; ia += va; }
+      const int vc = __shfl_up(ic, o, 64), va = __shfl_up(ia, o, 64), vg = __shfl_up(ig, o, 64);
+      if (lane >= o) { ic += vc; ia += va; ig += vg; }
     }
-    if (lane == 63) { part[wv] = ic; part[nt + wv] = ia; }
+    if (lane == 63) { part[wv] = ic; part[nt + wv] = ia; part[2 * nt - 1 - wv] = ig; }
     __syncthreads();
-    int oc = 0, oa = 0;   // the earlier waves' totals
-    for (int w = 0; w < wv; ++w) { oc += part[w]; oa += part[nt + w]; }
+    int oc = 0, oa = 0, og = 0;   // the earlier waves' totals
+    for (int w = 0; w < wv; ++w) { oc += part[w]; oa += part[nt + w]; og += part[2 * nt - 1 - w]; }
     int tc = 0, ta = 0;
     for (int w = 0; w < nwv; ++w) { tc += part[w]; ta += part[nt + w]; }
-    int acc = oc + ic - sc, na = oa + ia - sa;   // exclusive prefixes
+    int acc = oc + ic - sc, na = oa + ia - sa, ng = og + ig - sg;   // exclusive prefixes
+    if (tiles && tid == nt - 1) tiles[0] = ng + sg;
     for (int e = e0; e < e0 + per && e < ne; ++e) {
       const int c = cnt[e];
       cur[e] = acc;
@@ -365,6 +375,12 @@ __global__ __launch_bounds__(256) void kq4_moe_prep_kernel(
         rec[KQ4_MOE_REC * na + 1] = acc;
         rec[KQ4_MOE_REC * na + 2] = c;
         slt[e] = na++;
+        if (tiles)   // the grouped GEMM's: expert, offset of the tile's pairs, their count
+          for (int o = 0; o < c; o += 32, ++ng) {
+            tiles[1 + 4 * ng] = e;
+            tiles[2 + 4 * ng] = acc + o;
+            tiles[3 + 4 * ng] = c - o < 32 ? c - o : 32;
+          }
       }
       acc += c;
     }
@@ -379,9 +395,13 @@ __global__ __launch_bounds__(256) void kq4_moe_prep_kernel(
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       if (ev[j] >= 0 && ev[j] < ne) place(ev[j], tid + nt * j);
-    for (int i = tid + 4 * nt; i < n_pairs; i += nt) {
-      const int e = sel[i];
-      if (e >= 0 && e < ne) place(e, i);
+    for (int i0 = tid + 4 * nt; i0 < n_pairs; i0 += 8 * nt) {
+      int v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = i0 + nt * j < n_pairs ? sel[i0 + nt * j] : -1;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (v[j] >= 0 && v[j] < ne) place(v[j], i0 + nt * j);
     }
     return;
   }
@@ -1167,20 +1187,36 @@ int kq4_launch_moe_dbg(float *Y, const float *X, const int *sel, const float *pr
   // one token: every slot is a rank with one pair, the kernels take sel directly (no prep)
   const bool t1 = T == 1;
   const int slots = t1 ? tk : (ne < n_pairs ? ne : n_pairs);
+  // enough pairs per expert: both projections as grouped GEMMs
+  const bool gemm = !t1 && kq4_moe_gemm_ok(T, tk, ne, d, ef);
   if (!t1)
     hipLaunchKernelGGL(kq4_moe_prep_kernel, dim3((unsigned)(1 + (qblk + 7) / 8)), dim3(256),
-                       (3 * ne + 2 * 256) * sizeof(int), s, ws.ex_off, ws.ex_pair, ws.rec, slots,
-                       sel, n_pairs, ne, X, ws.xq, ws.xd, T, d);
+                       (3 * ne + 2 * 256) * sizeof(int), s, ws.ex_off, ws.ex_pair, ws.rec,
+                       gemm ? ws.tiles : nullptr, slots, sel, n_pairs, ne, X, ws.xq, ws.xd, T, d);
   const size_t lds_gu = (size_t)nst * kq4_moe_slab(16, KQ4_MOE_PCG) +
                         2 * KQ4_MOE_PCG * 32 * sizeof(float) +
                         (t1 ? (size_t)2 * 32 * (16 * nst + 1) * sizeof(float) : 0);   // T1 terms
-  hipLaunchKernelGGL(t1 ? kq4_moe_gu_kernel<true> : kq4_moe_gu_kernel<false>,
-                     dim3((unsigned)(slots * cbe)), dim3(128 * nst), lds_gu, s, G, U, ws.xq, ws.xd,
-                     ws.rec, ws.ex_pair, ws.avq, ws.avd, g_out, u_out, av_out, d, ef, tk, sel, X, ne);
+  if (gemm) {
+    const int e = kq4_launch_moe_gemm(0, G, U, ws, T, tk, ne, d, ef, g_out, u_out, av_out, s);
+    if (e) return e;
+  } else {
+    hipLaunchKernelGGL(t1 ? kq4_moe_gu_kernel<true> : kq4_moe_gu_kernel<false>,
+                       dim3((unsigned)(slots * cbe)), dim3(128 * nst), lds_gu, s, G, U, ws.xq,
+                       ws.xd, ws.rec, ws.ex_pair, ws.avq, ws.avd, g_out, u_out, av_out, d, ef, tk,
+                       sel, X, ne);
+  }
   if (av_in) {
     const long nblk = (long)n_pairs * cbe;
     hipLaunchKernelGGL(kq4_moe_avq_kernel, dim3((unsigned)((nblk + 7) / 8)), dim3(256), 0, s,
                        av_in, ws.avq, ws.avd, nblk);
+  }
+  if (gemm) {
+    const int e = kq4_launch_moe_gemm(1, D, D, ws, T, tk, ne, d, ef, nullptr, nullptr, nullptr, s);
+    if (e) return e;
+    const long n = (long)T * d;
+    hipLaunchKernelGGL(kq4_moe_combine_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, Y,
+                       ws.P, sel, pr, T, tk, d, ne);
+    return (int)hipGetLastError();
   }
   // one token with an even band (every band starts on a stream unit) and at most 16 ranks: down
   // and combine in one launch

@@ -188,6 +188,42 @@ def test_moe_invalid_expert_ids_skipped(kq4, torch_dev, orc, T):
     assert r <= 1e-5
 
 
+# The grouped GEMM (10 pairs per expert on average): tiles of 1, 31, 32, 33 and 64 pairs, an expert
+# without pairs, ids to skip; row sets that do not fill a workgroup, one and several stream stages.
+@pytest.mark.parametrize("counts,skip,tk,d,ef", [([1, 31, 32, 33], 0, 1, 64, 64),
+                                                 ([0, 64, 65, 7], 2, 2, 320, 448),
+                                                 ([40, 9, 3], 1, 1, 1088, 576),
+                                                 ([97, 1, 0, 31], 3, 4, 512, 1088)])
+def test_moe_grouped_gemm(kq4, torch_dev, orc, counts, skip, tk, d, ef):
+    torch = torch_dev
+    ne = len(counts)
+    ids = np.repeat(np.arange(ne), counts).tolist() + [-1, ne + 1, 2 * ne][:skip]
+    assert len(ids) % tk == 0 and len(ids) >= 10 * ne
+    rng = np.random.default_rng(d + ef)
+    sel = rng.permutation(ids).astype(np.int32).reshape(-1, tk)
+    T = len(sel)
+    pr = rng.random((T, tk)).astype(np.float32)
+    G, U, D = synth.make_moe(dict(hidden=d, experts=ne, top_k=tk, ef=ef), 60)
+    X = synth.make_activations(T, d, 61)
+    ok = (sel.reshape(-1) >= 0) & (sel.reshape(-1) < ne)
+    Y_o, st = orc.moe_ffn(X, sel, pr, G, U, D, ne, d, ef, stages=True)
+    dG, dU = (kq4.prepare_dev(to_dev(torch, a), ne * ef, d) for a in (G, U))
+    dD = kq4.prepare_dev(to_dev(torch, D), d, ne * ef)
+    dX, dsel, dpr = to_dev(torch, X), to_dev(torch, sel), to_dev(torch, pr)
+    Y, Y2 = (torch.empty((T, d), dtype=torch.float32, device="cuda") for _ in range(2))
+    gate, up, av = (torch.zeros((T * tk, ef), dtype=torch.float32, device="cuda") for _ in range(3))
+    kq4.moe_ffn_stages_dev(Y, dX, dsel, dpr, dG, dU, dD, ne, d, ef, gate=gate, up=up, av=av)
+    av_o = np.ascontiguousarray(st["av"])
+    av_o[~ok] = 0
+    kq4.moe_ffn_stages_dev(Y2, dX, dsel, dpr, dG, dU, dD, ne, d, ef, av_in=to_dev(torch, av_o))
+    torch.cuda.synchronize()
+    for got, want in ((gate, st["gate"]), (up, st["up"])):
+        assert np.array_equal(host(got)[ok].view(np.uint32), want[ok].view(np.uint32))
+    assert ulps(host(av)[ok], st["av"][ok]) <= 4
+    assert rel_err(host(Y), Y_o)[0] <= 1e-5   # as in check_stages: av's last ulps can move a code
+    assert np.array_equal(host(Y2).view(np.uint32), Y_o.view(np.uint32))
+
+
 def make_router(ne, d, seed):
     return (np.random.default_rng(seed).standard_normal((ne, d)) * 0.02).astype(np.float32)
 
