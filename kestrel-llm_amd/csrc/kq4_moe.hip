@@ -28,7 +28,7 @@
 #include "kq4_internal.h"
 
 #include <stdlib.h>
-#include <type_traits>
+#include <utility>
 
 #define KQ4_MOE_MAXTK 32
 #define KQ4_MOE_MAXNE 2048  // routing: a lane's experts fit one 32-bit mask
@@ -285,10 +285,152 @@ __global__ __launch_bounds__(320) void kq4_moe_logits_kernel(float *__restrict__
   if (adder && e0 + threadIdx.x < ne) logits[(size_t)t * ne + e0 + threadIdx.x] = s;
 }
 
+// Many tokens: the same chains, a lane per (token, expert) with its products formed in the lane. A
+// workgroup takes 64 tokens (a wave's lanes) and E experts (its waves). x goes through LDS as
+// [column / 4][token][4] tiles of 128 columns (double-buffered, loaded a tile ahead). A wave's
+// router weights are 16 to a register, the same in every row of 16 lanes, and each multiply takes
+// its own by a DPP row broadcast (as scalar operands they came through the scalar cache at a line
+// per ~40 cycles: 39 us). Bound by the two VALU instructions per product: 2048 columns x 128
+// experts at 1024 tokens 147 us -> 24.9 us, at 256 tokens 39.7 us -> 18.6 us.
+#define KQ4_RB_C 128       // columns per tile
+#define KQ4_RB_P 65        // LDS pitch of four columns (float4s): the transposing stores' banks differ
+
+typedef float kq4_f4 __attribute__((ext_vector_type(4)));
+
+// x * lane N's w of the row of 16 lanes
+template <int N>
+KQ4_DEV float kq4_mul_bcast(float w, float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(w), 0x150 + N, 0xf, 0xf,
+                                                    true)) * x;
+}
+
+// f(integral_constant<int, 0>), .., f(integral_constant<int, N - 1>)
+template <class F, int... I>
+KQ4_DEV void kq4_steps(F f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
+template <int E>
+__global__ __launch_bounds__(64 * E) void kq4_moe_logits_tiled_kernel(
+    float *__restrict__ logits, const float *__restrict__ router, const float *__restrict__ X,
+    int T, int ne, int d) {
+  extern __shared__ __align__(16) kq4_f4 kq4_rb_lds[];   // [2][KQ4_RB_C / 4][KQ4_RB_P]
+  constexpr int NQ = KQ4_RB_C / 4, NL = NQ / E, NW = KQ4_RB_C / 16;
+  // an XCD takes consecutive (token group, expert group) items: the groups of a token share its L2
+  const int n = gridDim.x, xcd = blockIdx.x & 7, q8 = n >> 3, r8 = n & 7;
+  const int it = xcd * q8 + (xcd < r8 ? xcd : r8) + (blockIdx.x >> 3);
+  const int neg = (ne + E - 1) / E;
+  const int t0 = 64 * (it / neg), lane = threadIdx.x & 63;
+  const int e = E * (it % neg) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lr = threadIdx.x / NQ, lq = threadIdx.x % NQ;   // loads: token lr + 64/NL j, columns 4 lq
+  // buffer loads: the tile's offset is scalar; columns past the last row's end read as zero
+  const int rows = min(T - t0, 64);
+  const auto rx = kq4_rsrc(X + (size_t)t0 * d, (uint32_t)(rows * d) * 4u);
+  const auto rr = kq4_rsrc(router + (size_t)(e < ne ? e : ne - 1) * d, (uint32_t)d * 4u);
+  kq4_f4 in[NL];
+  float w[NW];
+  uint32_t vx[NL];
+#pragma unroll
+  for (int j = 0; j < NL; ++j) vx[j] = (uint32_t)(min(lr + 64 / NL * j, rows - 1) * d + 4 * lq) * 4u;
+  const uint32_t vw = (uint32_t)(lane & 15) * 4u;
+  auto load = [&](int k) {
+#pragma unroll
+    for (int j = 0; j < NL; ++j)
+      in[j] = __builtin_bit_cast(kq4_f4, __builtin_amdgcn_raw_buffer_load_b128(
+                                             rx, vx[j], k * KQ4_RB_C * 4, 0));
+  };
+  auto load_w = [&](int j, int k) {
+    w[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                         rr, vw, min(k * KQ4_RB_C + 16 * j, d - 16) * 4, 0));
+  };
+  auto store = [&](int k) {
+#pragma unroll
+    for (int j = 0; j < NL; ++j)
+      kq4_rb_lds[((k & 1) * NQ + lq) * KQ4_RB_P + lr + 64 / NL * j] = in[j];
+  };
+  // Units of 16 columns: while unit u's products are added one after the other, u + 1's are formed
+  // (between the adds, each of which waits for the one before) and u + 2's x is on its way.
+  kq4_f4 x[2][4], p[2][4];
+  auto request = [&](int u) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[u & 1][j] = kq4_rb_lds[((u & (2 * NW - 1)) * 4 + j) * KQ4_RB_P + lane];
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  float s = 0.0f;
+  auto step = [&](auto odd, float wu) {   // unit of parity odd is added; wu is the next unit's
+    constexpr int O = decltype(odd)::value;
+    __builtin_amdgcn_s_waitcnt(0xc47f);   // lgkmcnt(4): x of unit u + 1, one wait for its 16 columns
+    kq4_steps([&](auto i) {
+      constexpr int I = decltype(i)::value;
+      s = s + p[O][I / 4][I % 4];
+      p[1 - O][I / 4][I % 4] = kq4_mul_bcast<I>(wu, x[1 - O][I / 4][I % 4]);
+      __builtin_amdgcn_sched_barrier(0);
+    }, std::make_integer_sequence<int, 16>{});
+  };
+  constexpr auto even = std::integral_constant<int, 0>{};
+  constexpr auto odd = std::integral_constant<int, 1>{};
+  load(0);
+#pragma unroll
+  for (int j = 0; j < NW; ++j) load_w(j, 0);
+  store(0);
+  __syncthreads();
+  request(0);
+  request(1);
+  kq4_steps([&](auto i) {
+    constexpr int I = decltype(i)::value;
+    p[0][I / 4][I % 4] = kq4_mul_bcast<I>(w[0], x[0][I / 4][I % 4]);
+  }, std::make_integer_sequence<int, 16>{});
+  load_w(0, 1);
+  const int nu = d / 16;
+  int u = 0;
+  for (; u + NW < nu; u += NW) {   // straight-line: a branch would let the loads sink to the stores
+    const int k = u / NW;
+    load(k + 1);
+#pragma unroll
+    for (int j = 0; j < NW; j += 2) {
+      if (j == NW - 2) {   // the next tile: its buffer was last read before this tile's barrier
+        store(k + 1);
+        __syncthreads();
+      }
+      request(u + j + 2);
+      step(even, w[j + 1]);
+      load_w(j + 1, k + 1);
+      request(u + j + 3);
+      step(odd, w[(j + 2) % NW]);
+      load_w((j + 2) % NW, j + 2 < NW ? k + 1 : k + 2);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NW; j += 2)   // the last tile (units past the row are read and not added)
+    if (u + j < nu) {
+      request(u + j + 2);
+      step(even, w[j + 1]);
+      request(u + j + 3);
+      step(odd, w[(j + 2) % NW]);
+    }
+  if (e < ne && t0 + lane < T) logits[(size_t)(t0 + lane) * ne + e] = s;
+}
+
 int kq4_launch_moe_logits(float *logits, const float *router, const float *X, int T, int ne,
                           int d, hipStream_t s) {
   if (T <= 0) return 0;
   if (d % 32) return (int)hipErrorInvalidValue;
+  // The token's own kernel runs 512 workgroups at a time (two per CU) and takes 10-12 us a round at 2048
+  // columns; the tiled one takes 18.5 us up to 256 workgroups of 4 experts. 96 tokens x 128
+  // experts 20.0 against 18.5 us, 192 x 60 19.9 against 18.6, 512 x 16 (1024 columns, one round) 8.0
+  // against 10.3. With more than 256, 8 experts share an x tile: 1024 x 128 28.0 -> 24.9 us.
+  if ((long)T * ((ne + KQ4_RT_E - 1) / KQ4_RT_E) > 512) {
+    const long tg = (T + 63) / 64, wg4 = tg * ((ne + 3) / 4);
+    const bool e4 = wg4 <= 256;
+    const unsigned grid = (unsigned)(e4 ? wg4 : tg * ((ne + 7) / 8));
+    const size_t lds = 2 * (KQ4_RB_C / 4) * KQ4_RB_P * sizeof(kq4_f4);
+    static std::atomic<unsigned long long> attr[2];   // 65 KB of LDS
+    auto k = e4 ? kq4_moe_logits_tiled_kernel<4> : kq4_moe_logits_tiled_kernel<8>;
+    const hipError_t err = kq4_lds_limit_once(reinterpret_cast<const void *>(k), (int)lds, attr[e4]);
+    if (err != hipSuccess) return (int)err;
+    hipLaunchKernelGGL(k, dim3(grid), dim3(e4 ? 256 : 512), lds, s, logits, router, X, T, ne, d);
+    return (int)hipGetLastError();
+  }
   const size_t lds = (2 * KQ4_RT_E * KQ4_RT_P + 32) * sizeof(float);
   static std::atomic<unsigned long long> attr{0};   // 66 KB of LDS
   hipError_t e = kq4_lds_limit_once(reinterpret_cast<const void *>(&kq4_moe_logits_kernel),

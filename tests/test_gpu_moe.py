@@ -241,6 +241,14 @@ def test_router_logits_bit_exact(kq4, torch_dev, orc, T, ne, d):
     assert np.array_equal(host(lg).view(np.uint32), want.view(np.uint32))
 
 
+# the tiled kernel: 4 and 8 experts a workgroup with the last group partial, 1 to 4 chunks in the
+# last tile, a single tile, tokens past the last group of 64
+@pytest.mark.parametrize("T,ne,d", [(129, 65, 32), (193, 41, 160), (513, 3, 192), (577, 9, 96),
+                                    (1025, 67, 128), (640, 130, 288), (70, 511, 512)])
+def test_router_logits_many_tokens(kq4, torch_dev, orc, T, ne, d):
+    test_router_logits_bit_exact(kq4, torch_dev, orc, T, ne, d)
+
+
 @pytest.mark.parametrize("T", [1, 64])
 @pytest.mark.parametrize("shape", ["small", "qwen3_30b_a3b"])
 def test_moe_layer_dev(kq4, torch_dev, orc, shape, T):
