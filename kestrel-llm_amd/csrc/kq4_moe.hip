@@ -194,7 +194,11 @@ __global__ __launch_bounds__(256) void kq4_moe_route_kernel(int *__restrict__ se
 // loads 8 float4s of one row (256 B apart) and the matching x (issued a tile ahead, so the loads
 // are in flight during a whole tile's 512 dependent adds, ~1.6 us), multiplies and stores the products
 // to LDS (double-buffered; row pitch 516 floats, so the adders' 16-B reads hit distinct banks);
-// each adder then adds its row's products in order.
+// each adder then adds its row's products in order. A dependent add takes 4.2 cycles and any other
+// instruction of the adder wave as much again, s_waitcnt included, so it waits once per 32 columns
+// and not per read, and issues ahead of the producers: 2048 columns x 128 experts at 1 token
+// 9.8 -> 8.5 us, at 64 tokens 11.5 -> 10.3 us. (A chain's products held in the lanes of a row and
+// added by DPP, without LDS: 12.8 us, each dependent DPP add needs two wait states.)
 #define KQ4_RT_E 16        // experts (chains) per workgroup
 #define KQ4_RT_C 512       // columns per tile
 #define KQ4_RT_P 516       // LDS row pitch (floats)
@@ -243,6 +247,7 @@ __global__ __launch_bounds__(320) void kq4_moe_logits_kernel(float *__restrict__
   if (wave > 0) load(0);
   float s = 0.0f;
   const bool adder = wave == 0 && threadIdx.x < KQ4_RT_E;
+  if (wave == 0) __builtin_amdgcn_s_setprio(3);   // its adds before the producers' work
   for (int k = 0; k < ntile; ++k) {
     if (wave > 0) {
       store(k);
@@ -263,6 +268,8 @@ __global__ __launch_bounds__(320) void kq4_moe_logits_kernel(float *__restrict__
         __builtin_amdgcn_sched_barrier(0);   // issued here, not sunk below the adds
       };
       auto add = [&](const float4 *v) {
+        asm volatile("" ::"v"(v[7].w));      // one wait for the chunk, not one per read
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           s += v[j].x;
@@ -270,6 +277,7 @@ __global__ __launch_bounds__(320) void kq4_moe_logits_kernel(float *__restrict__
           s += v[j].z;
           s += v[j].w;
         }
+        __builtin_amdgcn_sched_barrier(0);
       };
       rd(va, 0);
       int i = 0;
@@ -415,10 +423,11 @@ int kq4_launch_moe_logits(float *logits, const float *router, const float *X, in
                           int d, hipStream_t s) {
   if (T <= 0) return 0;
   if (d % 32) return (int)hipErrorInvalidValue;
-  // The token's own kernel runs 512 workgroups at a time (two per CU) and takes 10-12 us a round at 2048
-  // columns; the tiled one takes 18.5 us up to 256 workgroups of 4 experts. 96 tokens x 128
-  // experts 20.0 against 18.5 us, 192 x 60 19.9 against 18.6, 512 x 16 (1024 columns, one round) 8.0
-  // against 10.3. With more than 256, 8 experts share an x tile: 1024 x 128 28.0 -> 24.9 us.
+  // The token's own kernel runs 512 workgroups at a time (two per CU) and takes 8.5-10.4 us a round at
+  // 2048 columns; the tiled one takes 18.3 us up to 256 workgroups of 4 experts. Past the first
+  // round, 65 tokens x 128 experts 16.4 against 18.3 us, 96 x 128 17.9 against 18.3, 128 x 128 19.2
+  // against 18.4; 1024 columns x 16 experts at 512 tokens (one round) 7.3 against 10.0, at 600 10.7
+  // against 10.0. With more than 256, 8 experts share an x tile: 1024 x 128 28.0 -> 24.9 us.
   if ((long)T * ((ne + KQ4_RT_E - 1) / KQ4_RT_E) > 512) {
     const long tg = (T + 63) / 64, wg4 = tg * ((ne + 3) / 4);
     const bool e4 = wg4 <= 256;
