@@ -146,38 +146,29 @@ __global__ __launch_bounds__(256) void kq4_moe_route_kernel(int *__restrict__ se
     }
     return best;
   };
-  uint64_t mine = local_best();
-  int sk[KQ4_MOE_MAXTK];
-  float vk[KQ4_MOE_MAXTK];
-#pragma unroll
-  for (int k = 0; k < KQ4_MOE_MAXTK; ++k) {
-    if (k >= tk) break;
-    const uint64_t key = kq4_wave_max_u64(mine);
-    const int be = key ? (int)(0xFFFFFFFFu - (uint32_t)key) : -1;
-    sk[k] = be;
-    vk[k] = be >= 0 ? kq4_route_val(key) : -INFINITY;   // the logit, until the pass below
-    if (be >= 0 && (be & 63) == lane) {
-      taken |= 1u << (be >> 6);
-      mine = local_best();
-    }
-  }
-  // softmax over the k picks: lane k forms p_k = fl(exp(l_k - max)) (the picks are the same in
-  // every lane), the p_k are summed in rank order (lane reads), lane k writes fl(p_k * fl(1/sum))
+  // Rounds in a loop, lane k keeping pick k: unrolled to KQ4_MOE_MAXTK with the picks in arrays, every
+  // round ran its own copy of local_best and waited for its instructions (128 experts, top-8, kernel
+  // time: 1 token 5.4 -> 4.5 us, 64 tokens 6.2 -> 5.3, 1024 tokens 6.4 -> 5.4)
+  uint64_t mine = 0;
+  bool stale = true;   // the lane's best is taken
   float mx = -INFINITY, lk = -INFINITY;
   int sid = -1;
-#pragma unroll
-  for (int k = 0; k < KQ4_MOE_MAXTK; ++k) {
-    if (k >= tk) break;
-    mx = vk[k] > mx ? vk[k] : mx;
-    if (lane == k) { lk = vk[k]; sid = sk[k]; }
+  for (int k = 0; k < tk; ++k) {
+    if (stale) mine = local_best();
+    const uint64_t key = kq4_wave_max_u64(mine);
+    const int be = key ? (int)(0xFFFFFFFFu - (uint32_t)key) : -1;
+    const float v = be >= 0 ? kq4_route_val(key) : -INFINITY;
+    mx = v > mx ? v : mx;
+    if (lane == k) { lk = v; sid = be; }
+    stale = be >= 0 && (be & 63) == lane;
+    if (stale) taken |= 1u << (be >> 6);
   }
+  // softmax over the k picks: lane k forms p_k = fl(exp(l_k - max)), the p_k are summed in rank order
+  // (lane reads), lane k writes fl(p_k * fl(1/sum))
   const float pk = lane < tk ? kq4_expf(lk - mx) : 0.0f;
   float sum = 0.0f;
-#pragma unroll
-  for (int k = 0; k < KQ4_MOE_MAXTK; ++k) {
-    if (k >= tk) break;
+  for (int k = 0; k < tk; ++k)
     sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pk), k));
-  }
   const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
   if (lane < tk) {
     sel[(size_t)t * tk + lane] = sid;
