@@ -94,6 +94,16 @@ int cur_dev(DevState **out) {
 
 size_t grow_size(size_t bytes) { return al256(bytes > 4096 ? bytes + bytes / 4 : 4096); }
 
+// hipMalloc, false when refused. A refusal leaves no error behind: the runtime keeps a thread's last
+// error whatever succeeds after it, and every launcher returns hipGetLastError(), so the next launch
+// would report it as its own.
+bool dev_malloc(void **p, size_t bytes) {
+  if (hipMalloc(p, bytes) == hipSuccess) return true;
+  (void)hipGetLastError();
+  *p = nullptr;
+  return false;
+}
+
 // Staging buffers of the host-pointer API, whose calls are synchronous and cannot be captured
 // (they copy from and to host memory): grown by freeing the old buffer once the device is idle.
 int ensure(Buf &b, size_t bytes) {
@@ -105,10 +115,7 @@ int ensure(Buf &b, size_t bytes) {
     b.p = nullptr;
     b.cap = 0;
   }
-  if (hipMalloc(&b.p, n) != hipSuccess) {
-    b.p = nullptr;
-    return fail(KQ4_ENOMEM, "hipMalloc(%zu) failed", n);
-  }
+  if (!dev_malloc(&b.p, n)) return fail(KQ4_ENOMEM, "hipMalloc(%zu) failed", n);
   b.cap = n;
   return KQ4_OK;
 }
@@ -139,7 +146,7 @@ int ensure_ws(const Ws &ws, size_t payload, hipStream_t s) {
                 "is being captured; call kq4_workspace_reserve before capturing", bytes, b.cap);
   const size_t n = grow_size(bytes);
   void *p = nullptr;
-  if (hipMalloc(&p, n) != hipSuccess) return fail(KQ4_ENOMEM, "hipMalloc(%zu) failed", n);
+  if (!dev_malloc(&p, n)) return fail(KQ4_ENOMEM, "hipMalloc(%zu) failed", n);
   if (b.p) ws.ds->retired.push_back(b.p);
   b.p = p;
   b.cap = n;
@@ -671,7 +678,7 @@ int dev_weights(DevState *ds, uint64_t wkey, const uint8_t *w, int rows, int col
   uint8_t *dst = nullptr;
   if (wkey) {
     void *p = nullptr;
-    if (hipMalloc(&p, sbytes) != hipSuccess) return fail(KQ4_ENOMEM, "weights %zu B", sbytes);
+    if (!dev_malloc(&p, sbytes)) return fail(KQ4_ENOMEM, "weights %zu B", sbytes);
     dst = static_cast<uint8_t *>(p);
   } else {
     if ((rc = ensure(tmp, sbytes))) return rc;

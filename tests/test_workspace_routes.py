@@ -1,0 +1,154 @@
+"""The host side of the matmul calls without a GPU: which kernels a call launches and what it asks
+of the allocator, when the workspace can grow, cannot (memory full) or must not (a capturing
+stream). libkq4.so runs on a stand-in for the HIP runtime (tests/c/hip_standin.c): memory is
+addresses nobody reads, a launch is a line in a log. Planned for a 256-CU MI355X. The outputs of
+both forms of the prefill GEMM are compared on the GPU (test_gpu_matmul.py, test_gpu_graph.py)."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PKG = os.path.join(ROOT, "kestrel-llm_amd")
+
+PRELUDE = """
+import ctypes, json, sys
+sys.modules["torch"] = None       # its libraries would bind to the stand-in too
+hip = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+hip.standin_limit.argtypes = [ctypes.c_size_t]
+hip.standin_used.restype = ctypes.c_size_t
+hip.standin_log.restype = ctypes.c_char_p
+sys.path.insert(0, sys.argv[2])
+import kq4
+k = kq4.lib()
+assert k.kq4_init(0) == 0, kq4.last_error()
+BASE = 1 << 40                    # "device" addresses, far apart; host ones are never read either
+
+def at(i):
+    return BASE + (i << 36)
+
+def ptrs(n, first):
+    return (ctypes.c_void_p * n)(*[at(first + i) for i in range(n)])
+
+def call(form, n, rows, cols, chain=0):
+    \"\"\"One device call of `form` over the matrices of `rows`: (return code, kernels, hipMallocs).\"\"\"
+    hip.standin_clear()
+    before, m = hip.standin_mallocs(), len(rows)
+    r = (ctypes.c_int * m)(*rows)
+    outs, ws, x = ptrs(m, 1), ptrs(m, 8), at(0)
+    if form == "x":
+        rc = k.kq4_matmul_multi_dev(m, outs, None, ws, r, cols, x, n, chain, None)
+    elif form == "q":
+        rc = k.kq4_matmul_multi_q_dev(m, outs, None, ws, r, cols, x, at(16), n, chain, None)
+    elif form == "silu":
+        rc = k.kq4_matmul_silu_dev(at(1), x, at(16), None, at(8), rows[0], cols, n, chain, None)
+    elif form == "norm":
+        rc = k.kq4_rmsnorm_matmul_multi_dev(m, outs, None, ws, r, cols, x, at(16), 1e-6, 1, None, n,
+                                            chain, None)
+    elif form == "q8":
+        rc = k.kq4_q8_matmul_multi_dev(m, outs, None, ws, r, cols, x, n, chain, None)
+    elif form == "noalloc":
+        rc = k.kq4_matmul_noalloc_dev(at(1), x, None, at(8), rows[0], cols, n, chain, None)
+    lines = hip.standin_log().decode().split("\\n")[:-1]
+    return rc, [s.split(" ")[0] for s in lines], hip.standin_mallocs() - before
+
+def records(kernels):
+    return any("kq4_gemm_rec_kernel" in s for s in kernels)
+
+def token_major(kernels):
+    return any("kq4_gemm_kernel" in s for s in kernels)
+
+def up(b):
+    return (b + 255) // 256 * 256
+
+def need(form, n, rows, cols):
+    \"\"\"Workspace bytes of the token-major form: codes, scales and the partial sums of K splits.\"\"\"
+    main = n if form == "q8" else n & ~3
+    part = max((kq4.gemm_plan(n, r, cols, q8=form == "q8", ncu=256)[1] - 1) * main * r * 4
+               for r in rows)
+    return up(n * cols) + up(n * cols // 8) + up(part)
+
+def reserve_exactly(b):           # growth takes a quarter more than asked
+    b = (4 * b + 4) // 5
+    assert k.kq4_workspace_reserve(b) == 0
+"""
+
+
+@pytest.fixture(scope="module")
+def standin(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("standin") / "hip_standin.so")
+    r = subprocess.run(["gcc", "-std=gnu11", "-O1", "-Wall", "-Wextra", "-Werror", "-fPIC", "-shared",
+                        "-I/opt/rocm/include", os.path.join(ROOT, "tests", "c", "hip_standin.c"),
+                        "-o", so], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+
+    def run(body, **args):
+        """`body` in a process of its own on the stand-in; returns what it leaves in `result`."""
+        prog = PRELUDE + "".join(f"{n} = {v!r}\n" for n, v in args.items()) + body + \
+            "\nprint('RESULT ' + json.dumps(result))\n"
+        env = {n: v for n, v in os.environ.items() if not n.startswith("KQ4_")}
+        p = subprocess.run([sys.executable, "-c", prog, so, PKG], capture_output=True, text=True,
+                           env=env, timeout=120)
+        assert p.returncode == 0, p.stdout + p.stderr
+        line = [s for s in p.stdout.splitlines() if s.startswith("RESULT ")]
+        return json.loads(line[-1][7:])
+    return run
+
+
+# calls the record form takes when the workspace holds the records, which need more than the token-major
+# form: whole 64-token groups (520 tokens, 1000), and after the norm, beside the codes it wrote
+REC_CALLS = [("x", 520, [12288], 4096), ("silu", 520, [4096], 12288),
+             ("norm", 1024, [4096, 1024, 1024], 4096), ("q8", 1000, [12288], 4096)]
+
+
+@pytest.mark.parametrize("form,n,rows,cols", REC_CALLS)
+def test_full_memory_takes_the_token_major_form(standin, form, n, rows, cols):
+    """Memory that holds the token-major operands and not the records: the call runs token-major, as
+    it does in a workspace that was large enough before. hipMalloc's refusal, which the runtime keeps
+    as the thread's last error, is not taken for a failed launch."""
+    res = standin("""
+reserve_exactly(need(form, n, rows, cols))
+hip.standin_limit(hip.standin_used())
+full = call(form, n, rows, cols)
+hip.standin_limit(1 << 40)
+assert k.kq4_workspace_reserve(kq4.matmul_workspace_bytes(n, cols)) == 0
+room = call(form, n, rows, cols)
+result = [full[0], token_major(full[1]), records(full[1]), room[0], records(room[1])]
+""", form=form, n=n, rows=rows, cols=cols)
+    assert res[:3] == [0, True, False]        # done, token-major
+    assert res[3:] == [0, True]               # the same call with room: records
+
+
+def test_refused_allocation_does_not_fail_the_next_call(standin):
+    """A call that fails for lack of memory says so, and the next call, whose workspace fits, runs."""
+    res = standin("""
+assert k.kq4_workspace_reserve(1 << 20) == 0
+hip.standin_limit(hip.standin_used())
+big = call("x", 4096, [4096], 12288)
+small = call("x", 6, [4096], 4096, 0)
+result = [big[0], big[1], small[0], len(small[1]) > 0]
+""")
+    assert res == [-3, [], 0, True]           # KQ4_ENOMEM with nothing launched; then done
+
+
+def test_refused_weight_upload_does_not_fail_the_next_call(standin):
+    """The same for the host-pointer calls' buffers: an upload without memory for its device copy, one
+    without memory for the staging, then a device call that needs none."""
+    res = standin("""
+import numpy as np
+w = np.zeros(1024 * 128 * 72, np.uint8)       # 4096 x 4096
+assert k.kq4_workspace_reserve(1 << 20) == 0
+room = hip.standin_used()
+hip.standin_limit(room)
+a = k.kq4_weights_upload(1 << 32, w.ctypes.data, 4096, 4096)      # no staging
+b = call("x", 6, [4096], 4096)
+hip.standin_limit(room + w.size + w.size // 4 + 4096)
+c = k.kq4_weights_upload(1 << 32, w.ctypes.data, 4096, 4096)      # staging, no copy
+d = call("x", 6, [4096], 4096)
+hip.standin_limit(1 << 40)
+e = k.kq4_weights_upload(1 << 32, w.ctypes.data, 4096, 4096)
+result = [a, b[0], c, d[0], e]
+""")
+    assert res == [0, 0, 0, 0, 1]
