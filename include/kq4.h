@@ -39,6 +39,11 @@
  * call's own stream is asked whether it is capturing: a call that grows the workspace on
  * another stream while some stream captures in hipStreamCaptureModeGlobal fails in hipMalloc
  * (KQ4_ENOMEM) and invalidates that capture, so reserve first in that mode too.
+ * The prefill GEMM prefers a form that needs more workspace (activation records; the sizes above
+ * include it). Where the workspace does not hold that and cannot grow to it (a capturing stream,
+ * full memory, the fixed scratch of kq4_matmul_noalloc_dev) the call is done in the form that needs
+ * less, with the same outputs; refused memory is asked for again once the workspace has grown or
+ * kq4_workspace_trim was called.
  *
  * Error convention: device-pointer calls return KQ4_OK (0) or a negative KQ4_E* code;
  * host-pointer drop-in calls return 1 (done on the GPU) or 0 (not done: the caller runs its

@@ -63,6 +63,7 @@ struct DevState {
   int ncu = 256;        // compute units (sizes the GEMV grid)
   Buf ws;    // device-API workspace: quantized activations, MoE routing and staging
   std::vector<void *> retired;   // outgrown device-API workspaces, freed by kq4_shutdown
+  size_t refused = SIZE_MAX;     // smallest workspace that memory had no room for (try_ws)
   Buf hx, hu, hres, hout, hw, hsel, hpr, hstage;   // staging for the host-pointer API
   std::unordered_map<uint64_t, WEntry> wcache;
   uint8_t *scratch = nullptr;   // this device's address of kq4_scratch (set by kq4_init)
@@ -126,15 +127,28 @@ struct Ws {
   DevState *ds;   // nullptr: fixed (never grows)
 };
 
+// A larger workspace in ws's place, the old one retired; false when memory has no room for it.
+bool grow_ws(const Ws &ws, size_t bytes) {
+  const size_t n = grow_size(bytes);
+  void *p = nullptr;
+  if (!dev_malloc(&p, n)) {
+    if (bytes < ws.ds->refused) ws.ds->refused = bytes;
+    return false;
+  }
+  if (ws.b->p) ws.ds->retired.push_back(ws.b->p);
+  *ws.b = Buf{p, n};
+  ws.ds->refused = SIZE_MAX;
+  return true;
+}
+
 // Makes ws hold at least `bytes`. A HIP graph captured around a device-API call keeps the
 // workspace address it was recorded with, so a workspace is never freed while the library runs:
 // growth allocates a larger one and retires the old one (freed by kq4_shutdown), which graphs
 // captured before the growth go on using. Growth needs hipMalloc, which stream capture does not
 // allow, so a call on a capturing stream that would grow the workspace fails with KQ4_EINVAL
 // before it launches anything (kq4_workspace_reserve sizes it beforehand).
-int ensure_ws(const Ws &ws, size_t payload, hipStream_t s) {
-  Buf &b = *ws.b;
-  const size_t bytes = payload;
+int ensure_ws(const Ws &ws, size_t bytes, hipStream_t s) {
+  const Buf &b = *ws.b;
   if (b.cap >= bytes) return KQ4_OK;
   if (!ws.ds)
     return fail(KQ4_EINVAL, "the call needs %zu B of workspace; its fixed buffer holds %zu B",
@@ -144,13 +158,22 @@ int ensure_ws(const Ws &ws, size_t payload, hipStream_t s) {
   if (cs != hipStreamCaptureStatusNone)
     return fail(KQ4_EINVAL, "the workspace must grow to %zu B (it holds %zu B) while the stream "
                 "is being captured; call kq4_workspace_reserve before capturing", bytes, b.cap);
-  const size_t n = grow_size(bytes);
-  void *p = nullptr;
-  if (!dev_malloc(&p, n)) return fail(KQ4_ENOMEM, "hipMalloc(%zu) failed", n);
-  if (b.p) ws.ds->retired.push_back(b.p);
-  b.p = p;
-  b.cap = n;
+  if (!grow_ws(ws, bytes)) return fail(KQ4_ENOMEM, "hipMalloc(%zu) failed", grow_size(bytes));
   return KQ4_OK;
+}
+
+// Whether ws holds `bytes`, growing it where it may: ensure_ws for a form that the call can do without,
+// so a refusal is no failure and says nothing. Full memory is not asked again for as much until the
+// workspace has grown or been trimmed (a refused hipMalloc on every call otherwise).
+bool try_ws(const Ws &ws, size_t bytes, hipStream_t s) {
+  if (ws.b->cap >= bytes) return true;
+  if (!ws.ds || bytes >= ws.ds->refused) return false;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return cs == hipStreamCaptureStatusNone && grow_ws(ws, bytes);
 }
 
 struct Carve {   // bump allocator over a workspace
@@ -391,8 +414,8 @@ int run_gemv(DevState *ds, const Ws &wsp, int n_mats, float *const *out, const f
 // with each matrix's tile then in pl[]: option gemm_kind 0 never, 1 always, else where every matrix's
 // launch is faster so (kq4_rec_tile); the operands must stay within the kernel's buffer offsets and
 // the workspace hold the records and `more` bytes. A workspace that cannot grow to that (a fixed
-// buffer, a capturing stream) is no error: the call then takes the token-major form, which needs less
-// and gives the same bits.
+// buffer, a capturing stream, full memory) is no error: the call then takes the token-major form, which
+// needs less and gives the same bits.
 bool rec_fits(const DevState *ds, const Ws &ws, int n_mats, const int *rows, int cols, int n, int wf,
               KQ4GemmPlan *pl, size_t more, hipStream_t s) {
   const int kind = opt(kGemmKind);
@@ -402,7 +425,7 @@ bool rec_fits(const DevState *ds, const Ws &ws, int n_mats, const int *rows, int
     if (opt(kGemmTile) > 0 && t[i] != pl[i].tile) t[i] = 0;   // a forced tile is taken as it is
     if (kind == 0 || !t[i] || !kq4_gemm_rec_ok(rows[i], cols, n, wf)) return false;
   }
-  if (ensure_ws(ws, al256(kq4_rec_bytes(n, cols)) + more, s) != KQ4_OK) return false;
+  if (!try_ws(ws, al256(kq4_rec_bytes(n, cols)) + more, s)) return false;
   for (int i = 0; i < n_mats; ++i) pl[i].tile = t[i];
   return true;
 }
@@ -751,6 +774,7 @@ void kq4_shutdown(void) {
     }
     for (void *p : s.retired) (void)hipFree(p);
     s.retired.clear();
+    s.refused = SIZE_MAX;
     for (auto &kv : s.wcache) (void)hipFree(kv.second.p);
     s.wcache.clear();
     s.ready = false;
@@ -784,6 +808,7 @@ int kq4_workspace_trim(void) {
   int rc = cur_dev(&ds);
   if (rc) return rc;
   std::lock_guard<std::mutex> lk(g_mu);
+  ds->refused = SIZE_MAX;   // memory may have room again
   if (ds->retired.empty()) return KQ4_OK;
   KQ4_HIP(hipDeviceSynchronize());   // work queued before the call may still read them
   hipError_t e = hipSuccess;

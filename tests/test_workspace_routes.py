@@ -152,3 +152,41 @@ e = k.kq4_weights_upload(1 << 32, w.ctypes.data, 4096, 4096)
 result = [a, b[0], c, d[0], e]
 """)
     assert res == [0, 0, 0, 0, 1]
+
+
+@pytest.mark.parametrize("form,n,rows,cols", REC_CALLS)
+def test_fallback_is_quiet(standin, form, n, rows, cols):
+    """A call done token-major for want of workspace is no failure: it leaves the last failure's text
+    alone, with memory full and on a capturing stream. Full memory is asked once: later calls leave
+    the allocator alone until the workspace has grown or kq4_workspace_trim gave memory back."""
+    res = standin("""
+reserve_exactly(need(form, n, rows, cols))
+call("x", -5, [64], 64)
+text = kq4.last_error()
+hip.standin_capture(1)
+cap = call(form, n, rows, cols)
+hip.standin_capture(0)
+hip.standin_limit(hip.standin_used())
+full = [call(form, n, rows, cols) for _ in range(3)]
+same = kq4.last_error() == text
+hip.standin_limit(1 << 40)
+assert k.kq4_workspace_trim() == 0
+room = call(form, n, rows, cols)
+result = [same, "-5" in text, [cap[0], records(cap[1]), cap[2]],
+          [[c[0], records(c[1]), c[2]] for c in full], [room[0], records(room[1]), room[2]]]
+""", form=form, n=n, rows=rows, cols=cols)
+    assert res == [True, True, [0, False, 0], [[0, False, 1], [0, False, 0], [0, False, 0]],
+                   [0, True, 1]]
+
+
+def test_noalloc_without_room_for_records_is_quiet(standin):
+    """kq4_matmul_noalloc_dev's fixed scratch holds 68 tokens x 460000 columns token-major, and not
+    the records of two 64-token groups with the K split's partial sums."""
+    res = standin("""
+call("x", -5, [64], 64)
+text = kq4.last_error()
+a = call("noalloc", 68, [2048], 460000)
+b = call("noalloc", 68, [2048], 320000)       # those fit
+result = [kq4.last_error() == text, a[0], records(a[1]), a[2], b[0], records(b[1]), b[2]]
+""")
+    assert res == [True, 0, False, 0, 0, True, 0]
