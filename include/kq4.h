@@ -203,7 +203,7 @@ int kq4_moe_ffn(float *Y, const float *X, const int *sel, const float *pr, int T
 /* ---- device-pointer API (stream-ordered, asynchronous) ----------------------------------- */
 
 /* Workspace bytes the device-pointer matmuls (kq4_matmul_dev, _multi_dev, _silu_dev,
- * kq4_rmsnorm_matmul_multi_dev and the q8 twins) need for n_batch tokens of cols columns, and
+ * kq4_rmsnorm_matmul_multi_dev and the q8 twins) need for up to n_batch tokens of cols columns, and
  * the MoE calls (kq4_moe_ffn_dev, kq4_moe_ffn_stages_dev, kq4_moe_layer_dev) for T tokens; 0 for
  * a bad shape. The workspace is shared: reserve the largest any call will need. Beyond 8 tokens
  * the matmul figure includes up to 24 MiB for the partial sums of a K-split GEMM (the planner's

@@ -191,6 +191,10 @@ struct Carve {   // bump allocator over a workspace
 size_t qa_bytes(int n, int cols) {
   return al256((size_t)n * cols) + al256((size_t)n * (cols / 32) * sizeof(float));
 }
+// Most tokens of a fused RMSNorm whose rows are written in fp32 for the GEMV to quantize: from 5 the norm
+// kernel's codes measured faster even where the GEMV would quantize in its own kernel (Qwen3-8B QKV,
+// M = 5 / 6 / 8: 11.1 / 11.1 / 11.1 against 11.5 / 11.9 / 12.7 us).
+const int kNormRowsMax = 4;
 // The operand bytes kq4_matmul_noalloc_dev's documented limit counts (17/8 of a byte per element).
 size_t noalloc_bytes(int n, int cols) {
   return al256((size_t)n * (cols / 32) * 64) + al256((size_t)n * (cols / 32) * sizeof(float));
@@ -784,9 +788,11 @@ void kq4_shutdown(void) {
 
 size_t kq4_matmul_workspace_bytes(int n_batch, int cols) {
   if (n_batch < 0 || cols <= 0 || cols % 32) return 0;
-  // quantized activations and the one-token RMSNorm row; beyond the GEMV's tokens the prefill GEMM's
-  // activation records and the planner's K-split partial sums, at most KQ4_SPLIT_PART_MAX
-  size_t n = qa_bytes(n_batch, cols) + al256((size_t)cols * sizeof(float));
+  // quantized activations and the fp32 rows of a fused RMSNorm, also of a smaller batch than n_batch;
+  // beyond the GEMV's tokens the prefill GEMM's activation records and the planner's K-split partial
+  // sums, at most KQ4_SPLIT_PART_MAX
+  const int nr = n_batch < kNormRowsMax ? n_batch : kNormRowsMax;
+  size_t n = qa_bytes(n_batch, cols) + al256((size_t)nr * cols * sizeof(float));
   if (n_batch > KQ4_GEMV_MAX_M) n += al256(kq4_rec_bytes(n_batch, cols)) + (size_t)KQ4_SPLIT_PART_MAX;
   return n;
 }
@@ -1064,10 +1070,7 @@ int kq4_rmsnorm_matmul_multi_dev(int n_mats, float *const *out, const float *con
   // quantizer launch instead (Qwen3-8B QKV from 5 tokens on), the norm kernel writes the codes
   // and saves that launch (M = 8 12.15 -> 10.48 us).
   bool fp32_path = false;
-  // up to 4 tokens: from 5 the norm kernel's codes measured faster even where the GEMV would
-  // quantize in its own kernel (Qwen3-8B QKV, M = 5 / 6 / 8: 11.1 / 11.1 / 11.1 against
-  // 11.5 / 11.9 / 12.7 us)
-  if (n_batch <= 4) {
+  if (n_batch <= kNormRowsMax) {
     const GemvPlan pl = plan_gemv(n_mats, rows, (cols / 32 + KQ4_STREAM_CB - 1) / KQ4_STREAM_CB,
                                   ds->ncu, n_batch);
     const long per_cu = ((long)pl.groups + ds->ncu - 1) / ds->ncu;

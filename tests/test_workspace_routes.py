@@ -190,3 +190,33 @@ b = call("noalloc", 68, [2048], 320000)       # those fit
 result = [kq4.last_error() == text, a[0], records(a[1]), a[2], b[0], records(b[1]), b[2]]
 """)
     assert res == [True, 0, False, 0, 0, True, 0]
+
+
+# the largest batch an engine reserves for: every GEMV batch, the 16-token kernel, the prefill GEMM
+@pytest.mark.parametrize("most", [1, 2, 3, 4, 5, 7, 8, 12, 16, 17, 68, 77, 300, 1000])
+def test_reserved_workspace_holds_every_call_up_to_it(standin, most):
+    """kq4_workspace_reserve(kq4_matmul_workspace_bytes(most, cols)), then calls of up to `most` tokens
+    on a capturing stream: none needs more, and each takes the kernels it takes with all the workspace
+    it may want. (The sizes are the largest K and, for the K splits' partial sums, few and many rows.)"""
+    res = standin("""
+cols = 4096
+def calls():
+    out = []
+    for n in sorted({1, 2, 3, 4, 5, 6, 8, 9, 16, 17, 33, 67, 130, 1000, most - 1, most}):
+        if n < 1 or n > most:
+            continue
+        for rows in ([12288, 12288], [4096, 1024, 1024], [256]):
+            for form in ("x", "q", "silu", "norm", "q8"):
+                for c in (cols, 2080):
+                    out.append([form, n, rows, c, *call(form, n, rows[:1] if form == "silu" else rows, c)])
+    return out
+assert k.kq4_workspace_reserve(kq4.matmul_workspace_bytes(most, cols)) == 0
+reserve_only = hip.standin_used()
+hip.standin_capture(1)
+got = calls()
+hip.standin_capture(0)
+assert k.kq4_workspace_reserve(1 << 32) == 0
+want = calls()
+result = [[g, w[4:]] for g, w in zip(got, want) if g[4:] != w[4:] or g[4] != 0]
+""", most=most)
+    assert res == []
