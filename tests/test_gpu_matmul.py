@@ -241,6 +241,60 @@ def test_gemm_records_match_token_major(kq4, torch_dev, q8, n, rows, cols, tile,
         assert np.array_equal(o.view(np.uint32), outs[0].view(np.uint32))
 
 
+# Powers of ten for the activations (a token each) and the weight scales (a row each): f16 block scales
+# of every kind - normal, subnormal, the smallest, zero; for the activations also past the largest f16
+# (1e8: infinite, as the chain's rounding makes them) and an all-zero block's 1e-10 / 127.
+TOKEN_GAINS = [1.0, 1e-3, 1e-4, 1e-5, 3e-7, 1e-9, 0.0, 1e4, 1e6, 1e8]
+ROW_SCALES = [0.02, 1e-4, 3e-5, 1e-6, 6e-8, 0.0, 1.0, 3e4, -0.02, -3e-6]
+
+
+def same_bits(a, b):
+    """Bit equality, any NaN taken for any other."""
+    return np.array_equal(np.where(np.isnan(a), 0, a.view(np.uint32)),
+                          np.where(np.isnan(b), 0, b.view(np.uint32))) and \
+        np.array_equal(np.isnan(a), np.isnan(b))
+
+
+@pytest.mark.parametrize("tile", [1, 2])
+@pytest.mark.parametrize("q8", [False, True])
+def test_gemm_records_scale_range(kq4, torch_dev, orc, q8, tile):
+    """The record form over the f16 range of both scales, each output's terms of one magnitude (a
+    token's blocks share a gain, a row's a scale) and, on the tokens past the gains, of mixed ones:
+    the oracle's bits and the token-major form's. The matrix unit forms wd * f16r(xd) there, so this
+    needs it to take subnormal f16 operands as they are."""
+    torch = torch_dev
+    n, rows, cols, g = 132, 136, 544, 4
+    nb = cols // 32
+    rng = np.random.default_rng(17 + tile)
+    gain = np.array([TOKEN_GAINS[i % len(TOKEN_GAINS)] for i in range(n)], np.float32)[:, None]
+    gain = np.repeat(gain, nb, 1)
+    gain[100:] = rng.choice(TOKEN_GAINS[:9], (n - 100, nb))
+    x = synth.make_activations(n, cols, 18).reshape(n, nb, 32) * gain[:, :, None]
+    x = np.ascontiguousarray(x.reshape(n, cols), np.float32)
+    w = synth.make_q8_weights(rows, cols, 19, g=g) if q8 else synth.make_q4_weights(rows, cols, 19)
+    sc = np.array([ROW_SCALES[r % len(ROW_SCALES)] for r in range(rows)], np.float32)
+    sc = np.repeat(sc.reshape(rows // g, 1, g), nb, 1) * rng.uniform(0.5, 1.0, (rows // g, nb, g))
+    w[:, :, :2 * g] = sc.astype(np.float16).view(np.uint8).reshape(rows // g, nb, 2 * g)
+    res = synth.make_activations(n, rows, 20)
+    if q8:
+        want = orc.q8_matmul(w, x, rows, cols, residual=res, chain=kq4.CHAIN_Q8GEMM, g=g)
+        W = kq4.q8_prepare_dev(w, rows, cols, g=g)
+    else:
+        want = orc.matmul(w, x, rows, cols, residual=res, chain=kq4.CHAIN_ASM)
+        W = wdev(kq4, torch, w, rows, cols)
+    assert np.isfinite(want[gain.max(1) < 1e7]).all() and not np.isfinite(want).all()
+    got = []
+    for kind in (0, 1):
+        o = torch.full((n, rows), float("nan"), dtype=torch.float32, device="cuda")
+        with kq4.options(gemm_kind=kind, gemm_tile=tile, gemm_split=1):
+            (kq4.q8_matmul_dev if q8 else kq4.matmul_dev)(
+                o, to_dev(torch, x), W, rows, cols, residual=to_dev(torch, res),
+                chain=kq4.CHAIN_Q8GEMM if q8 else kq4.CHAIN_ASM)
+        got.append(host(o))
+    bad = [[t for t in range(n) if not same_bits(o[t], want[t])] for o in got]
+    assert bad == [[], []], "tokens off the oracle: token-major, records"
+
+
 @pytest.mark.parametrize("form", ["matmul", "silu", "multi"])
 def test_gemm_f8_auto_tail(kq4, torch_dev, orc, form):
     """The fp8-operand GEMM (gemm_kind = 1) with an AUTO-chain tail: 301 tokens are 300 on fp8

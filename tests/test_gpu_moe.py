@@ -224,6 +224,49 @@ def test_moe_grouped_gemm(kq4, torch_dev, orc, counts, skip, tk, d, ef):
     assert np.array_equal(host(Y2).view(np.uint32), Y_o.view(np.uint32))
 
 
+def test_moe_grouped_gemm_scale_range(kq4, torch_dev, orc):
+    """The grouped GEMM over wide ranges of both block scales (a token's gain, a weight row's scale:
+    f16 subnormal, the smallest, zero, negative): gate and up have the oracle's bits, and the down
+    projection of the oracle's av too."""
+    torch = torch_dev
+    ne, tk, d, ef, T = 4, 2, 320, 448, 60
+    gains = np.array([1.0, 1e-4, 1e-8, 1e-12, 0.0, 1e3], np.float32)
+    scales = np.array([0.02, 3e-5, 1e-6, 6e-8, 0.0, 1.0, -0.02, -3e-6], np.float32)
+    rng = np.random.default_rng(63)
+    G, U, D = synth.make_moe(dict(hidden=d, experts=ne, top_k=tk, ef=ef), 64)
+    for t in (G, U, D):
+        q, nb, _ = t.shape
+        sc = scales[rng.integers(0, len(scales), (q, 1, 4))] * rng.uniform(0.5, 1.0, (q, nb, 4))
+        t[:, :, :8] = sc.astype(np.float16).view(np.uint8).reshape(q, nb, 8)
+    X = synth.make_activations(T, d, 65) * gains[np.arange(T) % len(gains)][:, None]
+    sel = np.stack([rng.permutation(ne)[:tk] for _ in range(T)]).astype(np.int32)
+    pr = rng.random((T, tk)).astype(np.float32)
+    Y_o, st = orc.moe_ffn(X, sel, pr, G, U, D, ne, d, ef, stages=True)
+    assert np.isfinite(Y_o).all()
+    dG, dU = (kq4.prepare_dev(to_dev(torch, a), ne * ef, d) for a in (G, U))
+    dD = kq4.prepare_dev(to_dev(torch, D), d, ne * ef)
+    Y = torch.empty((T, d), dtype=torch.float32, device="cuda")
+    gate, up = (torch.zeros((T * tk, ef), dtype=torch.float32, device="cuda") for _ in range(2))
+    kq4.moe_ffn_stages_dev(Y, to_dev(torch, X), to_dev(torch, sel), to_dev(torch, pr), dG, dU, dD, ne, d,
+                           ef, gate=gate, up=up, av_in=to_dev(torch, st["av"]))
+    torch.cuda.synchronize()
+    for got, want in ((gate, st["gate"]), (up, st["up"]), (Y, Y_o)):
+        assert np.array_equal(host(got).view(np.uint32), want.view(np.uint32))
+
+
+# 128 experts at 6 and more pairs each on average: the whole FFN through the grouped GEMM
+@pytest.mark.parametrize("T", [97, 200])
+def test_moe_grouped_gemm_128_experts(kq4, torch_dev, orc, T):
+    check_stages(kq4, torch_dev, orc, dict(hidden=512, experts=128, top_k=8, ef=256), T, 66 + T,
+                 "128 experts")
+
+
+def test_moe_layer_grouped_gemm(kq4, torch_dev, orc):
+    """A prefill chunk through the whole layer at the Qwen3-30B-A3B shape: the tiled router logits and
+    the grouped GEMM (8.1 pairs per expert on average)."""
+    test_moe_layer_dev(kq4, torch_dev, orc, "qwen3_30b_a3b", 130)
+
+
 def make_router(ne, d, seed):
     return (np.random.default_rng(seed).standard_normal((ne, d)) * 0.02).astype(np.float32)
 
