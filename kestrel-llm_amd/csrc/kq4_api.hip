@@ -547,11 +547,16 @@ int matmul_impl(int n_mats, float *const *out, const float *const *res, const ui
   // tail tokens' codes; the other chains, and calls whose workspace cannot hold the records, on
   // token-major codes.
   const size_t base = x ? 0 : qbytes, tbytes = x && tail ? qa_bytes(tail, cols) : 0;
-  // (codes already quantized take one more launch to lay out, ~2.5 us, which the GEMM's gain of about
-  // 7 % covers from ~35 us on: 1.5e10 multiply-adds; Qwen3-8B QKV at 77 tokens, 1.9e9, lost 1.6 us)
+  // Codes already quantized take one more launch to lay out: ~2.5 us and ~0.4 us per million codes, as
+  // much as the GEMM gains on ~2048 rows of them. So what the rows beyond that gain, ~0.2 us per 1e9
+  // multiply-adds, has to cover the launch: from 1.3e10 on (us, token-major / records; 4096 x 12288 codes
+  // over 512 rows 76.0 / 93.7, 2048 x 8192 over 1024 55.0 / 61.0, 1024 x 4096 over 4096 51.0 / 53.7, a
+  // Qwen3-8B QKV at 77 tokens 1.6 more; 4096 x 2048 over 4096 94.3 / 90.7, 2048 x 4096 over 6144
+  // 136.8 / 117.9, 512 x 4096 over 12288 and 12288 135.9 / 126.4).
   long all_rows = 0;
   for (int i = 0; i < n_mats; ++i) all_rows += rows[i];
-  const bool gains = x || opt(kGemmKind) == 1 || (double)main_n * cols * all_rows >= 1.5e10;
+  const bool gains =
+      x || opt(kGemmKind) == 1 || (double)main_n * cols * (double)(all_rows - 2048) >= 1.3e10;
   if (main_chain == KQ4_CHAIN_ASM && gains &&
       rec_fits(ds, ws, n_mats, rows, cols, main_n, 0, pl, base + tbytes + pbytes, s)) {
     Carve cv{static_cast<char *>(ws.b->p), base};

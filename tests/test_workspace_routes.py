@@ -220,3 +220,24 @@ want = calls()
 result = [[g, w[4:]] for g, w in zip(got, want) if g[4:] != w[4:] or g[4] != 0]
 """, most=most)
     assert res == []
+
+
+# (form, tokens, rows, K) -> records: laying out codes that are already quantized (from the caller or the
+# norm) costs time in proportion to tokens x K, which few rows do not earn back
+@pytest.mark.parametrize("form,n,rows,cols,want", [
+    ("q", 4096, [512], 12288, False), ("q", 2048, [1024], 12288, False),
+    ("q", 4096, [1024, 512], 8192, False), ("norm", 4096, [512], 8192, False),
+    ("norm", 1024, [4096], 4096, False), ("q", 2048, [2048], 8192, False),
+    ("norm", 77, [4096, 1024, 1024], 4096, False),
+    ("q", 2048, [12288], 4096, True), ("norm", 2048, [12288, 12288], 4096, True),
+    ("norm", 2048, [4096, 1024, 1024], 4096, True), ("q", 4096, [4096], 4096, True),
+    ("x", 4096, [512], 12288, True), ("silu", 2048, [1024], 12288, True)])
+def test_record_layout_of_quantized_codes(standin, form, n, rows, cols, want):
+    res = standin("""
+assert k.kq4_workspace_reserve(1 << 32) == 0
+a = call(form, n, rows, cols)
+assert k.kq4_set_option(b"gemm_kind", 1) == 0
+b = call(form, n, rows, cols)
+result = [a[0], records(a[1]), token_major(a[1]), b[0], records(b[1])]
+""", form=form, n=n, rows=rows, cols=cols)
+    assert res == [0, want, not want, 0, True]
