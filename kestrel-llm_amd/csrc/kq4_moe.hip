@@ -414,12 +414,14 @@ int kq4_launch_moe_logits(float *logits, const float *router, const float *X, in
                           int d, hipStream_t s) {
   if (T <= 0) return 0;
   if (d % 32) return (int)hipErrorInvalidValue;
-  // The token's own kernel runs 512 workgroups at a time (two per CU) and takes 8.5-10.4 us a round at
-  // 2048 columns; the tiled one takes 18.3 us up to 256 workgroups of 4 experts. Past the first
-  // round, 65 tokens x 128 experts 16.4 against 18.3 us, 96 x 128 17.9 against 18.3, 128 x 128 19.2
-  // against 18.4; 1024 columns x 16 experts at 512 tokens (one round) 7.3 against 10.0, at 600 10.7
-  // against 10.0. With more than 256, 8 experts share an x tile: 1024 x 128 28.0 -> 24.9 us.
-  if ((long)T * ((ne + KQ4_RT_E - 1) / KQ4_RT_E) > 512) {
+  // The token's own kernel runs 512 workgroups at a time (two per CU) and is bound by its chains of adds,
+  // so a second round costs a whole one; the tiled one's time hardly depends on the workgroups up to
+  // 256 of 4 experts (with more, 8 experts share an x tile: 1024 tokens x 128 experts 28.0 -> 24.9 us) and
+  // grows with the columns at twice a round's slope. In us, own / tiled, at about 520, 896 and 1024
+  // workgroups: 512 columns 6.5, 8.1, 8.2 / 6.1; 1024 10.3, 12.5, 12.8 / 10.2; 2048 16.4, 18.6, 19.2 /
+  // 18.4; 3072 22.3, 24.6, 25.3 / 26.7; 4096 28.2, 30.7, 31.3 / 34.9; 8192 52.0, 55.4, 56.0 / 67.9; a
+  // third round (1088) 23.9 / 18.5 at 2048, 77.7 / 68.1 at 8192.
+  if ((long)T * ((ne + KQ4_RT_E - 1) / KQ4_RT_E) > (d >= 3072 ? 1024 : d >= 2048 ? 896 : 512)) {
     const long tg = (T + 63) / 64, wg4 = tg * ((ne + 3) / 4);
     const bool e4 = wg4 <= 256;
     const unsigned grid = (unsigned)(e4 ? wg4 : tg * ((ne + 7) / 8));

@@ -271,7 +271,9 @@ def make_router(ne, d, seed):
     return (np.random.default_rng(seed).standard_normal((ne, d)) * 0.02).astype(np.float32)
 
 
-@pytest.mark.parametrize("T,ne,d", [(1, 128, 2048), (7, 60, 96), (64, 128, 2048), (3, 300, 64)])
+# (the last three: a second round of workgroups in the few-token kernel, at its limits)
+@pytest.mark.parametrize("T,ne,d", [(1, 128, 2048), (7, 60, 96), (64, 128, 2048), (3, 300, 64),
+                                    (112, 128, 2048), (128, 127, 3104), (257, 60, 4096)])
 def test_router_logits_bit_exact(kq4, torch_dev, orc, T, ne, d):
     """fp32 router logits: the reference's serial chain per (token, expert), bit for bit."""
     torch = torch_dev

@@ -241,3 +241,18 @@ b = call(form, n, rows, cols)
 result = [a[0], records(a[1]), token_major(a[1]), b[0], records(b[1])]
 """, form=form, n=n, rows=rows, cols=cols)
     assert res == [0, want, not want, 0, True]
+
+
+# (tokens, experts, columns) -> the tiled router logits: past one round of the few-token kernel's
+# workgroups (512), past two where the columns are many
+@pytest.mark.parametrize("T,ne,d,want", [
+    (64, 128, 1024, False), (65, 128, 1024, True), (512, 16, 32, False), (513, 16, 32, True),
+    (65, 128, 2048, False), (96, 128, 2048, False), (112, 128, 2048, False), (113, 128, 2048, True),
+    (128, 128, 3072, False), (129, 128, 3072, True), (513, 8, 8192, False), (1024, 128, 2048, True)])
+def test_router_logits_kernel(standin, T, ne, d, want):
+    res = standin("""
+rc = k.kq4_moe_router_logits_dev(at(0), at(1), at(2), T, ne, d, None)
+result = [rc, hip.standin_log().decode()]
+""", T=T, ne=ne, d=d)
+    assert res[0] == 0 and res[1].count("\n") == 1
+    assert ("logits_tiled_kernel" in res[1]) == want
