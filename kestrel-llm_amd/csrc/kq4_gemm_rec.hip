@@ -213,7 +213,7 @@ __global__ __launch_bounds__(64 * WN, NW) void kq4_gemm_rec_kernel(
   "s_mov_b32 exec_hi, -1"
 #define KQ4_REC_ARGS                                                                            \
   ::"s"(l), "v"(v16), "v"(v4), "s"(ra), "s"(rx), "s"(rw), "s"(sx), "s"(sw), "s"(ss), "n"(XO),   \
-      "n"(WO), "n"(SO), "s"(sa), "n"(WO + 1024) : "memory"
+      "n"(WO), "n"(SO), "s"(sa), "n"(WO + 1024) : "memory", "m0"
     if constexpr (AP == 2 && WF == 0)
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
                    "buffer_load_dwordx4 %1, %3, %12 offen lds\n\t"

@@ -118,7 +118,7 @@ __global__ __launch_bounds__(256, 4) void kq4_moe_gemm_kernel(KQ4MoeGemmArgs a) 
         ::"s"(ldw + slot), "v"(va), "v"(vx), "v"(v16), "s"(ra), "s"(rx), "s"(rw0), "s"(rw1), "s"(sa),
         "s"(sx), "s"(b0w + cu), "s"(b1w + cu), "s"(b0w + cs + (WO0 - SO0)),
         "s"(b1w + cs + (WO1 - SO1)), "n"(XO), "n"(WO0), "n"(WO1), "n"(SO0), "n"(SO1)
-        : "memory");
+        : "memory", "m0");
   };
 
   const kq4_v16i zi = {0};
