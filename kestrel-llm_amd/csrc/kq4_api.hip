@@ -425,8 +425,10 @@ bool rec_fits(const DevState *ds, const Ws &ws, int n_mats, const int *rows, int
   const int kind = opt(kGemmKind);
   int t[KQ4_MAX_MATS];
   for (int i = 0; i < n_mats; ++i) {
-    t[i] = kind == 1 ? pl[i].tile : kq4_rec_tile(n, rows[i], wf, ds->ncu, pl[i]);
-    if (opt(kGemmTile) > 0 && t[i] != pl[i].tile) t[i] = 0;   // a forced tile is taken as it is
+    t[i] = kq4_rec_tile(n, rows[i], wf, ds->ncu, pl[i]);
+    if (kind == 1 && !t[i]) t[i] = wf ? 1 : 2;
+    if (opt(kGemmTile) > 0)   // a forced tile is taken as it is, where the form has it
+      t[i] = (kind == 1 || t[i] == pl[i].tile) && kq4_rec_has_tile(pl[i].tile, wf) ? pl[i].tile : 0;
     if (kind == 0 || !t[i] || !kq4_gemm_rec_ok(rows[i], cols, n, wf)) return false;
   }
   if (!try_ws(ws, al256(kq4_rec_bytes(n, cols)) + more, s)) return false;

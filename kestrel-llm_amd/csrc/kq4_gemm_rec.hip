@@ -143,7 +143,7 @@ __global__ __launch_bounds__(64 * WN, NW) void kq4_gemm_rec_kernel(
   constexpr int CBK = WF ? KQ8_STREAM_CB : KQ4_STREAM_CB;
   constexpr int CHK = WF ? KQ8_STREAM_CHUNK : KQ4_STREAM_CHUNK;
   constexpr int AP = GB * KB * 2 / WN;              // 1-KB code planes each wave brings in (1 or 2)
-  static_assert(AP == 1 || AP == 2, "kq4_gemm_rec_kernel: one record or half of one per wave");
+  static_assert(AP == 2 || (AP == 1 && WF == 0), "kq4_gemm_rec_kernel: a record or (q4) half of one per wave");
   // a wave's part of a stage in LDS: codes, their scales, its row set's scales and weights
   constexpr int XO = AP * 1024, SO = XO + KQ4_REC_X, WO = SO + 128, RW = WO + (WF ? 2048 : 1024);
   constexpr int SB = WN * RW, OPS = AP + (WF ? 4 : 3);   // a stage; its loads per wave
@@ -214,23 +214,19 @@ __global__ __launch_bounds__(64 * WN, NW) void kq4_gemm_rec_kernel(
 #define KQ4_REC_ARGS                                                                            \
   ::"s"(l), "v"(v16), "v"(v4), "s"(ra), "s"(rx), "s"(rw), "s"(sx), "s"(sw), "s"(ss), "n"(XO),   \
       "n"(WO), "n"(SO), "s"(sa), "n"(WO + 1024) : "memory", "m0"
-    if constexpr (AP == 2 && WF == 0)
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
-                   "buffer_load_dwordx4 %1, %3, %12 offen lds\n\t"
-                   "buffer_load_dwordx4 %1, %3, %12 offen offset:1024 lds\n\t" KQ4_REC_TAIL
-                   KQ4_REC_SC KQ4_REC_ARGS);
-    else if constexpr (AP == 2)
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
-                   "buffer_load_dwordx4 %1, %3, %12 offen lds\n\t"
-                   "buffer_load_dwordx4 %1, %3, %12 offen offset:1024 lds\n\t" KQ4_REC_TAIL
-                   "buffer_load_dwordx4 %1, %5, %7 offen offset:%13 lds\n\t" KQ4_REC_SC KQ4_REC_ARGS);
-    else if constexpr (WF == 0)
+    if constexpr (AP == 1)
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
                    "buffer_load_dwordx4 %1, %3, %12 offen lds\n\t" KQ4_REC_TAIL
+                   KQ4_REC_SC KQ4_REC_ARGS);
+    else if constexpr (WF == 0)
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
+                   "buffer_load_dwordx4 %1, %3, %12 offen lds\n\t"
+                   "buffer_load_dwordx4 %1, %3, %12 offen offset:1024 lds\n\t" KQ4_REC_TAIL
                    KQ4_REC_SC KQ4_REC_ARGS);
     else
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
-                   "buffer_load_dwordx4 %1, %3, %12 offen lds\n\t" KQ4_REC_TAIL
+                   "buffer_load_dwordx4 %1, %3, %12 offen lds\n\t"
+                   "buffer_load_dwordx4 %1, %3, %12 offen offset:1024 lds\n\t" KQ4_REC_TAIL
                    "buffer_load_dwordx4 %1, %5, %7 offen offset:%13 lds\n\t" KQ4_REC_SC KQ4_REC_ARGS);
 #undef KQ4_REC_TAIL
 #undef KQ4_REC_SC
@@ -373,6 +369,8 @@ static hipError_t rec_launch(float *out, const float *res, const uint8_t *w, con
   return hipGetLastError();
 }
 
+int kq4_rec_has_tile(int tile, int wf) { return tile == 1 || (tile == 2 && !wf); }
+
 int kq4_gemm_rec_ok(int rows, int cols, int n_tok, int wf) {
   return kq4_rec_bytes(n_tok, cols) < KQ4_OOB - 4096 &&
          (wf ? kq8_stream_bytes(rows, cols) : kq4_stream_bytes(rows, cols)) < KQ4_OOB - 4096;
@@ -389,15 +387,15 @@ int kq4_gemm_rec_ok(int rows, int cols, int n_tok, int wf) {
 //   * q4, unsplit: the tile of fewer rounds (8B gate 12288 x 4096 at M = 512, 64 x 128: 75.9 / 68.4;
 //     M = 768 and 2048, 128 x 128: 118.1 / 107.7, 267.8 / 232.3; QKV M = 2048 150.9 / 120.0);
 //   * q8: 128 x 128 only, split or from two tiles per CU (8B gate M = 768 / 1000 / 2048 137.2 / 127.5,
-//     162.7 / 143.3, 330.6 / 280.3; at M = 512, 384 tiles, 85.2 / 95.6; its 64 x 128 form, whose
-//     weights are twice the bytes, is slower throughout).
+//     162.7 / 143.3, 330.6 / 280.3; at M = 512, 384 tiles, 85.2 / 95.6; there is no 64 x 128 form:
+//     at twice the weight bytes it was slower throughout).
 int kq4_rec_tile(int n_tok, int rows, int wf, int ncu, const KQ4GemmPlan &plan) {
   const long cu = ncu < 1 ? 1 : ncu;
   const long t1 = (long)((n_tok + 127) / 128) * ((rows + 127) / 128);
   const long t2 = (long)((n_tok + 63) / 64) * ((rows + 127) / 128);
   if (wf) return plan.ksplit > 1 ? plan.tile == 1 : t1 >= 2 * cu;
   if (plan.tile == 3) return 0;
-  if (plan.ksplit > 1) return plan.tile;
+  if (plan.ksplit > 1) return kq4_rec_has_tile(plan.tile, wf) ? plan.tile : 0;
   const long r1 = (t1 + 3 * cu - 1) / (3 * cu), r2 = (t2 + 4 * cu - 1) / (4 * cu);
   return 100 * r1 <= 71 * r2 ? 1 : 2;
 }
@@ -407,16 +405,13 @@ int kq4_launch_gemm_rec(float *out, const float *res, const uint8_t *w, const ui
                         float *part, int prio) {
   if (n_tok <= 0 || rows <= 0) return 0;
   const int ks = kq4_split_len(cols / 32, wf ? KQ8_STREAM_CB : KQ4_STREAM_CB, ksplit);
-  if (!kq4_gemm_rec_ok(rows, cols, n_tok, wf) || ksplit < 1 || ksplit > KQ4_GEMM_SPLIT_MAX || !ks ||
-      (ksplit > 1 && !part))
+  if (!kq4_gemm_rec_ok(rows, cols, n_tok, wf) || !kq4_rec_has_tile(tile, wf) || ksplit < 1 ||
+      ksplit > KQ4_GEMM_SPLIT_MAX || !ks || (ksplit > 1 && !part))
     return (int)hipErrorInvalidValue;
-#define KQ4_REC(TM, WN, NW)                                                                        \
-  (wf ? rec_launch<TM, WN, 1, NW>(out, res, w, rec, rows, cols, n_tok, ksplit, ks, part, prio, s)  \
-      : rec_launch<TM, WN, 0, NW>(out, res, w, rec, rows, cols, n_tok, ksplit, ks, part, prio, s))
-  const hipError_t e = tile == 1 || tile == 4 ? KQ4_REC(4, 4, 3)
-                       : tile == 2            ? KQ4_REC(2, 4, 4)
-                                              : KQ4_REC(2, 2, 4);
-#undef KQ4_REC
+  const hipError_t e =
+      wf          ? rec_launch<4, 4, 1, 3>(out, res, w, rec, rows, cols, n_tok, ksplit, ks, part, prio, s)
+      : tile == 1 ? rec_launch<4, 4, 0, 3>(out, res, w, rec, rows, cols, n_tok, ksplit, ks, part, prio, s)
+                  : rec_launch<2, 4, 0, 4>(out, res, w, rec, rows, cols, n_tok, ksplit, ks, part, prio, s);
   if (e != hipSuccess || ksplit < 2) return (int)e;
   return kq4_launch_split_reduce(out, res, part, ksplit - 1, (long)n_tok * rows, s);
 }

@@ -135,6 +135,7 @@ int kq4_launch_quantize_rec(const float *x, const float *up, uint8_t *rec, int8_
 int kq4_launch_rec_from_q8(const int8_t *xq, const float *xd, uint8_t *rec, int n, int cols,
                            hipStream_t s);
 int kq4_gemm_rec_ok(int rows, int cols, int n_tok, int wf);   // within 32-bit buffer offsets
+int kq4_rec_has_tile(int tile, int wf);   // 128 x 128; q4 also 64 x 128
 // The record form's tile for a launch the planner runs as `plan` (its K slices are kept), or 0 where
 // the token-major form is faster.
 int kq4_rec_tile(int n_tok, int rows, int wf, int ncu, const KQ4GemmPlan &plan);

@@ -256,3 +256,46 @@ result = [rc, hip.standin_log().decode()]
 """, T=T, ne=ne, d=d)
     assert res[0] == 0 and res[1].count("\n") == 1
     assert ("logits_tiled_kernel" in res[1]) == want
+
+
+def test_forced_forms_of_the_records(standin):
+    """gemm_kind = 1 takes the record kernel for every ASM and Q8GEMM launch, at the forced tile where
+    there is one (gemm_tile) and the form has it: 128 x 128, q4 also 64 x 128. A tile it does not have
+    runs token-major, as do the other chains and gemm_kind = 0. The calls the GPU tests force
+    through it run it."""
+    from test_gpu_matmul import RECORD_EDGES
+    res = standin("""
+import re
+assert k.kq4_workspace_reserve(1 << 32) == 0
+
+def forced(form, n, rows, cols, chain, kind, tile, split=-1):
+    for o, v in ((b"gemm_kind", kind), (b"gemm_tile", tile), (b"gemm_split", split)):
+        assert k.kq4_set_option(o, v) == 0
+    rc, names, _ = call(form, n, rows, cols, chain)
+    assert rc == 0
+    m = re.search(r"kq4_gemm_rec_kernelILi(\\d)ELi4ELi(\\d)", " ".join(names))
+    return [64 * int(m[1]) // 2, int(m[2])] if m else None       # tokens of the tile, q8
+
+result = dict(
+    edges=[[forced("q8" if q8 else f, n, [rows], cols, 0, 1, 1 if q8 else tile, split)
+            for f in (["x"] if q8 else ["x", "q"])]
+           for n, rows, cols, tile, split in edges for q8 in (False, True)],
+    tiles=[[forced(f, 300, [2000], 672, c, kind, tile) for tile in (0, 1, 2, 3, 4)]
+           for f, c, kind in [("x", 3, 1), ("x", 0, 1), ("q8", 4, 1), ("x", 2, 1), ("x", 1, 1),
+                              ("q8", 2, 1), ("x", 3, 0), ("q8", 4, 0)]],
+    small=[forced("x", 24, [64], 256, 3, 1, 0), forced("q8", 24, [64], 256, 4, 1, 0),
+           forced("x", 24, [64], 256, 3, -1, 0)],
+    # a forced tile under the planner's choice of form, K split
+    split4=forced("x", 512, [4096], 12288, 3, -1, 4, 4))
+""", edges=RECORD_EDGES)
+    want = []
+    for n, rows, cols, tile, split in RECORD_EDGES:
+        want += [[[64 if tile == 2 else 128, 0]] * 2, [[128, 1]]]
+    assert res["edges"] == want
+    q4 = [[128, 0], [64, 0], None, None]
+    tm = [None] * 5
+    assert res["tiles"][0][1:] == q4 and res["tiles"][1][1:] == q4
+    assert res["tiles"][0][0] and res["tiles"][1][0]
+    assert res["tiles"][2] == [[128, 1], [128, 1], None, None, None]
+    assert res["tiles"][3:] == [tm] * 5
+    assert res["small"] == [[64, 0], [128, 1], None] and res["split4"] is None
