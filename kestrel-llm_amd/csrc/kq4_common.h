@@ -202,12 +202,19 @@ KQ4_DEV int kq4_dot4(uint32_t a, uint32_t b, int c) {
 
 // ---- raw buffer loads -------------------------------------------------------------------------
 // Loads through a buffer resource of `bytes` bytes: the hardware's range check returns zeros for
-// offsets at or past the end, so loads of tiles that overhang a matrix need no branches (an
-// offset of KQ4_OOB reads zeros too).
+// offsets at or past the end (the scalar offset counts: measured), so loads of tiles that overhang a
+// matrix need no branches (an offset of KQ4_OOB reads zeros too).
 #define KQ4_OOB 0xFFFFFFF0u
 KQ4_DEV __amdgpu_buffer_rsrc_t kq4_rsrc(const void *p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes,
                                            0x00020000);   // gfx9 raw buffer, 32-bit data
+}
+// The resource as a vector, for loads in inline assembly; its byte `off` is p's first (for loads with the
+// immediate offset `off`).
+typedef int kq4_rsrc4 __attribute__((ext_vector_type(4)));
+KQ4_DEV kq4_rsrc4 kq4_rsrc_at(const void *p, uint32_t bytes, uint32_t off) {
+  const uint64_t a = (uint64_t)(uintptr_t)p - off;
+  return kq4_rsrc4{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), (int)(bytes + off), 0x00020000};
 }
 KQ4_DEV uint4 kq4_bload16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);

@@ -126,13 +126,6 @@ int kq4_launch_rec_from_q8(const int8_t *xq, const float *xd, uint8_t *rec, int 
 // Operands of fp6 digits, whose MFMA gives the sum in fp32 without a convert, measured 230 us: 42 VALU
 // per block to unpack the weights' signs and magnitudes, 1.5 times the operand bytes, 1.9 GHz.
 
-typedef int kq4_rsrc4 __attribute__((ext_vector_type(4)));
-// A buffer resource whose byte `off` is p's first (for loads with the immediate offset `off`).
-KQ4_DEV kq4_rsrc4 kq4_rsrc_at(const void *p, uint32_t bytes, uint32_t off) {
-  const uint64_t a = (uint64_t)(uintptr_t)p - off;
-  return kq4_rsrc4{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), (int)(bytes + off), 0x00020000};
-}
-
 template <int TM, int WN, int WF, int NW>
 __global__ __launch_bounds__(64 * WN, NW) void kq4_gemm_rec_kernel(
     float *__restrict__ out, const float *__restrict__ res, const uint8_t *__restrict__ w,

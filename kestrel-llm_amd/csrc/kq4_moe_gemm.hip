@@ -9,13 +9,6 @@
 typedef int kq4_v4i __attribute__((ext_vector_type(4)));
 typedef int kq4_v16i __attribute__((ext_vector_type(16)));
 typedef float kq4_v32f __attribute__((ext_vector_type(32)));
-typedef int kq4_rsrc4 __attribute__((ext_vector_type(4)));
-
-// A buffer resource whose byte `off` is p's first (for loads with the immediate offset `off`).
-KQ4_DEV kq4_rsrc4 kq4_rsrc_at(const void *p, uint32_t bytes, uint32_t off) {
-  const uint64_t a = (uint64_t)(uintptr_t)p - off;
-  return kq4_rsrc4{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), (int)(bytes + off), 0x00020000};
-}
 
 struct KQ4MoeGemmArgs {
   const uint8_t *w0, *w1;   // the two matrices whose row sets a wave takes (G, U; D, D)
@@ -152,7 +145,8 @@ __global__ __launch_bounds__(256, 4) void kq4_moe_gemm_kernel(KQ4MoeGemmArgs a) 
     }
   };
   // lanes 0-31: the first row set's scales, 32-63: the second's. S comes as 16*S, so wd / 16: every
-  // step is scaled by a power of two far from underflow (wd >= 2^-24, xd >= 1e-10/127)
+  // step is scaled by a power of two far from underflow (wd >= 2^-24, xd >= 1e-10/127). (Where wd * xd
+  // itself overflows, activations beyond 6e35, a zero S gives 0 here and NaN in the chain.)
   auto set_w = [&](uint32_t s) { wv = kq4_h2f(s) * 0.0625f; };
   auto issue_s = [&](int q) {
     S[q & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[(q >> 1) & 1], bf[q & 1], zi, 0, 0, 0);
