@@ -1,6 +1,7 @@
 """The prefill GEMM planner (host logic, no GPU): the launch forms it picks for the measured
-shapes, and the invariants every pick keeps (kq4_gemm_plan_info, include/kq4.h). Planned for a
-256-CU MI355X."""
+shapes, and the invariants every pick keeps (kq4_gemm_plan_info, include/kq4.h). The plan is the
+token-major form's; the record form keeps its K slices and takes a tile of its own
+(test_workspace_routes.py: test_record_rule). Planned for a 256-CU MI355X."""
 import os
 
 import pytest

@@ -229,3 +229,36 @@ def test_graph_gemv_chunks_and_small_batch_split(kq4, torch_dev, orc):
         for n in xs:
             assert np.array_equal(out[n].cpu().numpy().view(np.uint32),
                                   want[n].view(np.uint32)), (rep, n)
+
+
+def test_graph_prefill_without_room_for_records(kq4, torch_dev, orc):
+    """A prefill call captured with a workspace that holds its token-major operands and not the
+    activation records it prefers (they are whole 64-token groups): the capture takes the token-major
+    form (test_workspace_routes.py) and every replay, with eager work between them, has the bits of the
+    eager call on records."""
+    torch = torch_dev
+    n, rows, cols = 200, 2048, 4096
+    w = synth.make_q4_weights(rows, cols, 61)
+    x = synth.make_activations(n, cols, 62)
+    W = kq4.prepare_dev(to_dev(torch, w), rows, cols)
+    X = to_dev(torch, x)
+    out, eager = (torch.empty((n, rows), device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    kq4.lib().kq4_shutdown()                  # drops the workspace other tests have grown
+    kq4.init(0)
+    split = kq4.gemm_plan(n, rows, cols)[1]
+    assert split > 1
+    need = n * cols + n * cols // 8 + (split - 1) * n * rows * 4   # codes, scales, partial sums
+    kq4.workspace_reserve((4 * need + 4) // 5)                     # growth takes a quarter more
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        kq4.matmul_dev(out, X, W, rows, cols, stream=torch.cuda.current_stream())
+    for rep in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        kq4.matmul_dev(eager, X, W, rows, cols)     # grows the workspace: on records
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), rep
+    e, _ = rel_err(out.cpu().numpy(), orc.matmul(w, x, rows, cols))
+    assert e <= 1e-5, e

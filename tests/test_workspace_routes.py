@@ -100,7 +100,8 @@ def standin(tmp_path_factory):
 # calls the record form takes when the workspace holds the records, which need more than the token-major
 # form: whole 64-token groups (520 tokens, 1000), and after the norm, beside the codes it wrote
 REC_CALLS = [("x", 520, [12288], 4096), ("silu", 520, [4096], 12288),
-             ("norm", 1024, [4096, 1024, 1024], 4096), ("q8", 1000, [12288], 4096)]
+             ("norm", 1024, [4096, 1024, 1024], 4096), ("q8", 1000, [12288], 4096),
+             ("x", 200, [2048], 4096)]        # (the one test_gpu_graph.py captures)
 
 
 @pytest.mark.parametrize("form,n,rows,cols", REC_CALLS)
@@ -180,13 +181,13 @@ result = [same, "-5" in text, [cap[0], records(cap[1]), cap[2]],
 
 
 def test_noalloc_without_room_for_records_is_quiet(standin):
-    """kq4_matmul_noalloc_dev's fixed scratch holds 68 tokens x 460000 columns token-major, and not
-    the records of two 64-token groups with the K split's partial sums."""
+    """kq4_matmul_noalloc_dev's fixed scratch (64 MiB) holds 68 tokens x 464384 columns token-major, and
+    not the records of their two 64-token groups with the K split's partial sums."""
     res = standin("""
 call("x", -5, [64], 64)
 text = kq4.last_error()
-a = call("noalloc", 68, [2048], 460000)
-b = call("noalloc", 68, [2048], 320000)       # those fit
+a = call("noalloc", 68, [128], 464384)
+b = call("noalloc", 68, [128], 460000)       # those fit
 result = [kq4.last_error() == text, a[0], records(a[1]), a[2], b[0], records(b[1]), b[2]]
 """)
     assert res == [True, 0, False, 0, 0, True, 0]
@@ -299,3 +300,25 @@ result = dict(
     assert res["tiles"][2] == [[128, 1], [128, 1], None, None, None]
     assert res["tiles"][3:] == [tm] * 5
     assert res["small"] == [[64, 0], [128, 1], None] and res["split4"] is None
+
+
+# (form, tokens, rows, K) -> tokens of the record kernel's tile, 0 = token-major: the shapes the rule's
+# comment gives figures for (Qwen3-8B gate, QKV and down, Qwen3-VL-2B gate, Q8_0 gate) and its edges
+RECORD_TILES = [
+    ("x", 512, 12288, 4096, 64), ("x", 768, 12288, 4096, 128), ("x", 2048, 12288, 4096, 128),
+    ("x", 2048, 6144, 4096, 128), ("x", 24, 6144, 4096, 0), ("x", 128, 6144, 2048, 0),
+    ("silu", 96, 4096, 12288, 64), ("silu", 256, 4096, 12288, 64), ("silu", 512, 4096, 12288, 128),
+    ("silu", 768, 4096, 12288, 64), ("q8", 512, 12288, 4096, 0), ("q8", 768, 12288, 4096, 128),
+    ("q8", 1000, 12288, 4096, 128), ("q8", 2048, 12288, 4096, 128), ("x", 64, 12288, 4096, 0)]
+
+
+@pytest.mark.parametrize("form,n,rows,cols,tile", RECORD_TILES)
+def test_record_rule(standin, form, n, rows, cols, tile):
+    res = standin("""
+import re
+assert k.kq4_workspace_reserve(1 << 32) == 0
+rc, names, _ = call(form, n, [rows], cols)
+m = re.search(r"kq4_gemm_rec_kernelILi(\\d)", " ".join(names))
+result = [rc, 32 * int(m[1]) if m else 0, token_major(names)]
+""", form=form, n=n, rows=rows, cols=cols)
+    assert res == [0, tile, tile == 0]

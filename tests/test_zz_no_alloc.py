@@ -5,8 +5,9 @@ through the C ABI, on two calls in a row (the second smaller, so it reads a scra
 holds the first call's data), on a one-token call (in-kernel quantization, no scratch) and on a
 shape too large for the scratch (refused before anything runs). It is captured in a HIP graph
 at the largest shape the scratch holds and every replay matches the eager kq4_matmul_dev bit for
-bit; the largest shapes also run the fp8-operand GEMM (option gemm_kind = 1), whose operands
-(n_batch * cols * 17/8 bytes) fill the scratch."""
+bit. Shapes are refused by n_batch * cols * 17/8 bytes; whole 64-token groups of activation records
+(36 bytes per token and block) with the K split's partial sums can still exceed the scratch, and then
+the call runs token-major: both sides of that line are run."""
 import numpy as np
 import pytest
 
@@ -51,8 +52,8 @@ def test_noalloc_matches_matmul_dev(kq4, torch_dev):
 
 def test_noalloc_largest_fits_and_beyond_is_refused(kq4, torch_dev):
     torch = torch_dev
-    # 2048 tokens x 12288 columns (the Qwen3-8B down prefill): 28.3 MB of int8 operands, and
-    # with gemm_kind = 1 53.5 MB of fp8 operands, within the 64 MiB scratch
+    # 2048 tokens x 12288 columns (the Qwen3-8B down prefill): 28.3 MB of operands in either form
+    # (gemm_kind = 1: records) and the K split's partial sums, within the 64 MiB scratch
     a, b = run_both(kq4, torch, 128, 12288, 2048, 41, residual=False)
     assert np.array_equal(bits(a), bits(b))
     with kq4.options(gemm_kind=1):
@@ -66,9 +67,17 @@ def test_noalloc_largest_fits_and_beyond_is_refused(kq4, torch_dev):
         kq4.matmul_noalloc_dev(out, x, w, rows, cols)
 
 
+# 68 tokens are two 64-token groups of records: 66.5 MB with the 8 slices' partial sums, which the 64 MiB
+# scratch (67.1 MB) holds, and 67.12 MB, which it does not (which form runs: test_workspace_routes.py)
+@pytest.mark.parametrize("cols", [460000, 464384])
+def test_noalloc_at_the_end_of_the_scratch(kq4, torch_dev, cols):
+    a, b = run_both(kq4, torch_dev, 128, cols, 68, 45, residual=True)
+    assert np.array_equal(bits(a), bits(b))
+
+
 def test_noalloc_under_graph_capture(kq4, torch_dev):
-    """2048 tokens x 15392 columns, first on int8 operands with the K-split partial sums in the
-    scratch, then on fp8 operands: 64 MiB less 128 KiB of scratch. torch
+    """2048 tokens x 15392 columns, 64 MiB less 128 KiB by the 17/8-byte limit, with the K-split partial
+    sums in the scratch: first as the planner runs it, then on records (gemm_kind = 1). torch
     captures in the global mode, in which HIP refuses a hipMalloc from any thread and the
     capture fails, so a capture that succeeds and replays shows that the call allocated
     nothing. The graph is replayed three times, with eager calls of other shapes in between that
@@ -81,7 +90,7 @@ def test_noalloc_under_graph_capture(kq4, torch_dev):
     x = to_dev(torch, synth.make_activations(n, cols, 52))
     res = to_dev(torch, synth.make_activations(n, rows, 53))
     got = torch.full((n, rows), float("nan"), dtype=torch.float32, device="cuda")
-    # the int8 form: 35.5 MB of operands and the K-split partial sums (16 tiles, 4 slices)
+    # 35.5 MB of operands and the K-split partial sums (16 tiles, 4 slices)
     g8 = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g8):
         kq4.matmul_noalloc_dev(got, x, w, rows, cols, residual=res,
