@@ -118,13 +118,13 @@ int kq4_launch_rec_from_q8(const int8_t *xq, const float *xd, uint8_t *rec, int 
 // issued before tile q's epilogue, its scale product after it, its fragments one tile earlier.
 // Against kq4_gemm_kernel (128 x 128, the ASM chain): 16 registers of scale products instead of 64
 // (f16 tiles instead of f32 outer products of two tiles) and none of staged loads, 149 instead of 239,
-// so three workgroups share a CU instead of two; Qwen3-8B gate 12288 x 4096 at M = 2048: 130 SIMD cycles
-// per tile instead of 197, 216 instead of 258 us (0.19 of int8 peak; the clock falls from 2.07 to
-// 1.99 GHz). What bounds it: the instructions of a tile in three waves (35 VALU at about 1.9 cycles
-// beside 36 cycles the two MFMAs keep to themselves; timing copies without the convert 99 cycles per
-// tile, without the scale product 19 less, without the loads 7 less), and the clock under that load.
-// Operands of fp6 digits, whose MFMA gives the sum in fp32 without a convert, measured 230 us: 42 VALU
-// per block to unpack the weights' signs and magnitudes, 1.5 times the operand bytes, 1.9 GHz.
+// so three workgroups share a CU instead of two (2.7 waves resident per SIMD instead of 1.9). Qwen3-8B gate
+// 12288 x 4096 at M = 2048: 158 SIMD cycles per tile and block instead of 196 (GRBM_GUI_ACTIVE, both at
+// 2.0 GHz), with the quantizer 228-234 instead of 263-268 us in graph replays (0.18 of int8 peak). What
+// bounds it: VALU issue. A wave issues 38 VALU instructions per tile and block, 32 of them the convert
+// and the fma per output; the SIMD issues one every 4.2 cycles, the matrix unit beside it is busy 40 %.
+// Operands of fp6 digits, whose MFMA gives the sum in fp32 without a convert, measured 6 % slower: 42
+// VALU per block to unpack the weights' signs and magnitudes, 1.5 times the operand bytes, a lower clock.
 
 template <int TM, int WN, int WF, int NW>
 __global__ __launch_bounds__(64 * WN, NW) void kq4_gemm_rec_kernel(

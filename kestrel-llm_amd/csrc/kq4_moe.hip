@@ -188,7 +188,8 @@ __global__ __launch_bounds__(256) void kq4_moe_route_kernel(int *__restrict__ se
 // each adder then adds its row's products in order. A dependent add takes 4.2 cycles and any other
 // instruction of the adder wave as much again, s_waitcnt included, so it waits once per 32 columns
 // and not per read, and issues ahead of the producers: 2048 columns x 128 experts at 1 token
-// 9.8 -> 8.5 us, at 64 tokens 11.5 -> 10.3 us. (A chain's products held in the lanes of a row and
+// 9.8 -> 8.5 us, at 64 tokens 11.5 -> 10.3 us (graph replays of the call alone, the router in the cache;
+// with 17 copies of it in turn 10.9 -> 9.8 and 12.5 -> 11.3 us). (A chain's products held in the lanes of a row and
 // added by DPP, without LDS: 12.8 us, each dependent DPP add needs two wait states.)
 #define KQ4_RT_E 16        // experts (chains) per workgroup
 #define KQ4_RT_C 512       // columns per tile
@@ -290,7 +291,8 @@ __global__ __launch_bounds__(320) void kq4_moe_logits_kernel(float *__restrict__
 // router weights are 16 to a register, the same in every row of 16 lanes, and each multiply takes
 // its own by a DPP row broadcast (as scalar operands they came through the scalar cache at a line
 // per ~40 cycles: 39 us). Bound by the two VALU instructions per product: 2048 columns x 128
-// experts at 1024 tokens 147 us -> 24.9 us, at 256 tokens 39.7 us -> 18.6 us.
+// experts at 1024 tokens 148 us -> 25 us, at 256 tokens 39.8 us -> 18.7 us (graph replays of the call
+// alone; 30 us in the kernel trace of a whole 1024-token layer).
 #define KQ4_RB_C 128       // columns per tile
 #define KQ4_RB_P 65        // LDS pitch of four columns (float4s): the transposing stores' banks differ
 

@@ -33,13 +33,13 @@ struct KQ4MoeGemmArgs {
 // fl(wd*xd) come from one v_mfma_f32_32x32x1_2b_f32 (its two blocks are the two row sets).
 // Loads go straight to LDS through a three-stage ring as in kq4_gemm_rec_kernel; a pair's activation
 // row is gathered there by its lane's address, so nothing is copied into expert order first.
-// Bound by the VALU work of the chain (a conversion, a multiply and an add per block, row and pair;
-// the products themselves keep the matrix unit a third as long), with a quarter of the tiles' pairs
-// padding at 64 pairs per expert on average. 32-pair tiles, not 64: with four accumulator tiles
+// Bound by the VALU work of the chain (a conversion, a multiply and an add per block, row and pair: a VALU
+// instruction every 4.6 SIMD cycles with 2.8 waves resident, the matrix unit busy 20 %), with a fifth of
+// the tiles' pairs padding at 64 pairs per expert on average. 32-pair tiles, not 64: with four accumulator tiles
 // and the scale products a wave needs more than 128 VGPRs and spills. Rings of 4 and 5 stages
-// (3 and 2 workgroups per CU) were 4% and 17% slower. Qwen3-30B-A3B's FFN at 1024 tokens (8192 pairs): gate/up
-// 482 us -> 146 us (177 TMAC/s) and down 148 us -> 79 us against kq4_moe.hip's kernels, which
-// unpack an expert's weights again for every 4 to 8 of its pairs and contract on v_dot4.
+// (3 and 2 workgroups per CU) were 4% and 17% slower. Qwen3-30B-A3B's FFN at 1024 tokens (8192 pairs, kernel
+// trace of the layer): gate/up 482 us -> 157 us (164 TMAC/s) and down 148 us -> 84 us against
+// kq4_moe.hip's kernels, which unpack an expert's weights again for every 4 to 8 of its pairs and contract on v_dot4.
 template <int DOWN>
 __global__ __launch_bounds__(256, 4) void kq4_moe_gemm_kernel(KQ4MoeGemmArgs a) {
   constexpr int KB = 2, NQ = 2 * KB;
