@@ -188,8 +188,8 @@ __global__ __launch_bounds__(256) void kq4_moe_route_kernel(int *__restrict__ se
 // each adder then adds its row's products in order. A dependent add takes 4.2 cycles and any other
 // instruction of the adder wave as much again, s_waitcnt included, so it waits once per 32 columns
 // and not per read, and issues ahead of the producers: 2048 columns x 128 experts at 1 token
-// 9.8 -> 8.5 us, at 64 tokens 11.5 -> 10.3 us (graph replays of the call alone, the router in the cache;
-// with 17 copies of it in turn 10.9 -> 9.8 and 12.5 -> 11.3 us). (A chain's products held in the lanes of a row and
+// 9.8 -> 8.5 us, at 64 tokens 11.5 -> 10.3 us (graphs of 40 calls;
+// of 17 calls, as the bench's, 10.9 -> 9.8 and 12.5 -> 11.3 us). (A chain's products held in the lanes of a row and
 // added by DPP, without LDS: 12.8 us, each dependent DPP add needs two wait states.)
 #define KQ4_RT_E 16        // experts (chains) per workgroup
 #define KQ4_RT_C 512       // columns per tile
